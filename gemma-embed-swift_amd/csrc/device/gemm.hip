@@ -139,6 +139,15 @@ struct GemmCfg {
 using GemmWide = GemmCfg<128, 256, 2, 4, 32, 3>;
 using GemmSquare = GemmCfg<256, 256, 4, 4, 64, 2>;
 using GemmSmall = GemmCfg<128, 128, 2, 2, 64, 2>;
+// Launches whose tiles of the shapes above would leave most of the CUs idle take smaller tiles and
+// deeper stage rings (one or two workgroups a CU, so the ring, not the neighbours, covers the
+// copies' latency); gemm_shape holds the rule and what it measured.
+using GemmMini = GemmCfg<64, 64, 2, 2, 128, 3>;
+using GemmMini64 = GemmCfg<64, 64, 2, 2, 64, 3>;
+using GemmMid = GemmCfg<64, 128, 2, 2, 64, 4>;
+using GemmDeep = GemmCfg<128, 128, 4, 2, 64, 3>;
+// The QKV projection's tile for those launches: 64 tokens of 256 / head_dim whole heads.
+using GemmQkvHalf = GemmCfg<64, 256, 2, 4, 64, 3>;
 // 256 x 192 tiles of 4 x 2 waves of 64 x 96 (three column fragments, so no GeGLU pairs), K in
 // stages of 64, two stages (112 KB): the 768-wide projections over many rows (768 = 4 x 192:
 // 256 tiles at 16384 rows, one per CU).
@@ -474,16 +483,14 @@ struct QkvStage {
     // 16-byte chunk c of row r at chunk c ^ (r % 16): the transposed fragment writes of one
     // instruction (32 rows, one chunk) and the V^T column reads spread over the banks.
     __device__ static constexpr int off(int r, int c) { return r * RB + ((c ^ (r & 15)) << 4); }
-    static constexpr int BYTES = 128 * RB;
 };
 
-template <int HD>
-__global__ __launch_bounds__(GemmWide::NT) __attribute__((amdgpu_waves_per_eu(4))) void gemm_qkv_kernel(const uint16_t* __restrict__ X,
+template <int HD, class C>
+__global__ __launch_bounds__(C::NT) __attribute__((amdgpu_waves_per_eu(4))) void gemm_qkv_kernel(const uint16_t* __restrict__ X,
                                                                  const uint16_t* __restrict__ Fh, int M, int N, int K,
                                                                  int tiles_n, int tiles, QkvEpilogue a) {
-    using C = GemmWide;
-    static_assert(C::BM == 128 && C::BN == 256 && 256 % HD == 0, "heads per tile");
-    static_assert(QkvStage::BYTES <= C::LDS, "staging fits the stage buffers");
+    static_assert(C::BM % 64 == 0 && C::BN == 256 && 256 % HD == 0, "heads per tile");
+    static_assert(C::BM * QkvStage::RB <= C::LDS, "staging fits the stage buffers");
     extern __shared__ __attribute__((aligned(1024))) unsigned char lds[];
     const int tile = xcd_tile(blockIdx.x, tiles);
     const int m0 = (tile / tiles_n) * C::BM, n0 = (tile % tiles_n) * C::BN;
@@ -568,8 +575,13 @@ __global__ __launch_bounds__(GemmWide::NT) __attribute__((amdgpu_waves_per_eu(4)
     if (tile_slot0 + 256 / HD <= first_v || tile_slot0 >= S) return;  // no V head in this tile
     wait_lgkmcnt0();
     workgroup_barrier();
-    const int t0 = m0 + lane, t1 = m0 + 64 + lane;
-    const int vc0 = t0 < M ? a.vcol[t0] : -1, vc1 = t1 < M ? a.vcol[t1] : -1;
+    constexpr int TG = C::BM / 64;  // 64-token groups of the tile
+    int vc[TG];
+#pragma unroll
+    for (int i = 0; i < TG; i++) {
+        const int t = m0 + 64 * i + lane;
+        vc[i] = t < M ? a.vcol[t] : -1;
+    }
     for (int hh = 0; hh < 256 / HD; hh++) {
         const int sl = tile_slot0 + hh;
         if (sl < first_v || sl >= S) continue;
@@ -577,10 +589,13 @@ __global__ __launch_bounds__(GemmWide::NT) __attribute__((amdgpu_waves_per_eu(4)
         for (int d = wave; d < HD; d += C::NW) {
             const int col = hh * HD + d;
             uint16_t* row = a.vt + (size_t)((sl - first_v) * HD + d) * a.vt_cols;
-            const uint16_t v0 = *reinterpret_cast<const uint16_t*>(lds + QkvStage::off(lane, col >> 3) + (col & 7) * 2);
-            const uint16_t v1 = *reinterpret_cast<const uint16_t*>(lds + QkvStage::off(64 + lane, col >> 3) + (col & 7) * 2);
-            if (vc0 >= 0) row[vc0] = v0;
-            if (vc1 >= 0) row[vc1] = v1;
+            uint16_t v[TG];
+#pragma unroll
+            for (int i = 0; i < TG; i++)
+                v[i] = *reinterpret_cast<const uint16_t*>(lds + QkvStage::off(64 * i + lane, col >> 3) + (col & 7) * 2);
+#pragma unroll
+            for (int i = 0; i < TG; i++)
+                if (vc[i] >= 0) row[vc[i]] = v[i];
         }
     }
 }
@@ -649,6 +664,13 @@ hipError_t gemm_configure_shape() {
     return e;
 }
 
+template <class C>
+hipError_t gemm_qkv_configure() {
+    hipError_t e = set_lds_limit(gemm_qkv_kernel<128, C>, C::LDS);
+    if (e == hipSuccess) e = set_lds_limit(gemm_qkv_kernel<256, C>, C::LDS);
+    return e;
+}
+
 // Workgroup slots of a GemmWide launch: two workgroups per CU (contexts may be created from
 // several threads; they all store the same device's count).
 static std::atomic<int> g_wide_slots{512};
@@ -662,8 +684,11 @@ hipError_t gemm_configure() {
     if (e == hipSuccess) e = gemm_configure_shape<GemmSquare>();
     if (e == hipSuccess) e = gemm_configure_shape<GemmSmall>();
     if (e == hipSuccess) e = gemm_configure_shape<GemmNarrow>();
-    if (e == hipSuccess) e = set_lds_limit(gemm_qkv_kernel<128>, GemmWide::LDS);
-    if (e == hipSuccess) e = set_lds_limit(gemm_qkv_kernel<256>, GemmWide::LDS);
+    if (e == hipSuccess) e = gemm_configure_shape<GemmMini>();
+    if (e == hipSuccess) e = gemm_configure_shape<GemmMid>();
+    if (e == hipSuccess) e = gemm_configure_shape<GemmDeep>();
+    if (e == hipSuccess) e = gemm_qkv_configure<GemmWide>();
+    if (e == hipSuccess) e = gemm_qkv_configure<GemmQkvHalf>();
     return e;
 }
 
@@ -751,8 +776,11 @@ hipError_t gemm_skinny_launch(hipStream_t s, const Q8Dev& w, const uint16_t* x, 
     return hipGetLastError();
 }
 
-// K / 16 must be a multiple of 8 (of 4 would do for the GeGLU pairs).
-bool skinny_ok(const Q8Dev& w, int M) { return M <= kSkinnyMaxRows && w.cols % 128 == 0; }
+// Whether a launch takes the skinny kernel: its 32-row blocks (of 32 columns, 64 for the GeGLU
+// pairs) are at most one wave per CU, and K / 16 is a multiple of 8 (of 4 would do for the pairs).
+bool skinny_ok(const Q8Dev& w, int M, int cols) {
+    return w.cols % 128 == 0 && int64_t((M + 31) / 32) * (w.rows / cols) <= g_wide_slots.load(std::memory_order_relaxed) / 2;
+}
 
 hipError_t launch_gemm_q8(hipStream_t s, const Q8Dev& w, const uint16_t* x, int M, void* y, GemmEpilogue epi,
                           float out_scale, const GemmEpiArgs* eap) {
@@ -767,7 +795,7 @@ hipError_t launch_gemm_q8(hipStream_t s, const Q8Dev& w, const uint16_t* x, int 
     }
     if (!gemm_operands_ok(w, x, M, y)) return hipErrorInvalidValue;
     if (M == 0) return hipSuccess;
-    if (skinny_ok(w, M)) {
+    if (skinny_ok(w, M, epi == kEpiGeglu ? 64 : 32)) {
         switch (epi) {
         case kEpiF32: return gemm_skinny_launch<kEpiF32, false, 1>(s, w, x, M, y, out_scale);
         case kEpiF16: return gemm_skinny_launch<kEpiF16, false, 1>(s, w, x, M, y, out_scale);
@@ -776,6 +804,25 @@ hipError_t launch_gemm_q8(hipStream_t s, const Q8Dev& w, const uint16_t* x, int 
         case kEpiHeads: return gemm_skinny_launch<kEpiHeads, false, 1>(s, w, x, M, y, out_scale, ea);
         default: return hipErrorInvalidValue;
         }
+    }
+    // Launches too small for the large tiles: the smallest tiles that are still at most one per CU
+    // (two for 64 x 64 with K in stages of 64: 48 KB), so that every CU has work and the ring of
+    // stages covers its copies. Measured alone on the chip at the encoders' projections, each launch
+    // reading another layer's weights (us, the shapes below against these): o 768 x 768
+    // 10.3 -> 5.1 at 1024 rows, 11.7 -> 6.7 at 2100, 11.3 -> 8.0 at 4096; down 768 x 1152
+    // 15.1 -> 6.2, 15.9 -> 8.9, 15.5 -> 10.3; down 512 x 2048 23.8 -> 8.8, 24.3 -> 12.6,
+    // 24.4 -> 13.7; gate/up 2304 x 768 12.7 -> 8.3 at 1024 and 12.8 -> 9.2 at 1600. Past one round
+    // of the 128 x 128 tiles the shapes below win again (gate/up at 2100 rows 13.0 against 13.9).
+    // The two parts of a split forward choose by their own rows: counting both parts' tiles was
+    // slower (a 4096-token pack 2.27 against 2.09 ms, 8192 3.60 against 3.42).
+    if (w.cols % 64 == 0) {
+        const int64_t cus = g_wide_slots.load(std::memory_order_relaxed) / 2;
+        const auto tiles = [&](int bm, int bn) { return int64_t((M + bm - 1) / bm) * ((w.rows + bn - 1) / bn); };
+        if (epi != kEpiGeglu && w.cols % GemmMini::BK == 0 && tiles(64, 64) <= cus)
+            return gemm_launch<GemmMini>(s, w, x, M, y, epi, out_scale, ea);
+        if (epi != kEpiGeglu && tiles(64, 64) <= cus * 7 / 4) return gemm_launch<GemmMini64>(s, w, x, M, y, epi, out_scale, ea);
+        if (tiles(64, 128) <= cus) return gemm_launch<GemmMid>(s, w, x, M, y, epi, out_scale, ea);
+        if (tiles(128, 128) <= cus) return gemm_launch<GemmDeep>(s, w, x, M, y, epi, out_scale, ea);
     }
     // Tile shapes by projection and batch rows, from sweeps of the shapes (20 launches back to
     // back, one box). The tile shape does not change the results: every shape runs the same MFMA
@@ -802,13 +849,24 @@ hipError_t launch_gemm_q8(hipStream_t s, const Q8Dev& w, const uint16_t* x, int 
 
 bool gemm_qkv_supported(int hd, int H, int KV) { return (hd == 128 || hd == 256) && H > 0 && KV > 0; }
 
+template <class C>
+hipError_t gemm_qkv_launch(hipStream_t s, const Q8Dev& w, const uint16_t* x, int M, int hd, const QkvEpilogue& e) {
+    const int N = w.rows, K = w.cols;
+    const int tiles_m = (M + C::BM - 1) / C::BM, tiles_n = (N + C::BN - 1) / C::BN, tiles = tiles_m * tiles_n;
+    if (hd == 128)
+        launch_kernel(gemm_qkv_kernel<128, C>, dim3(tiles), dim3(C::NT), C::LDS, s, x, w.fh, M, N, K, tiles_n, tiles, e);
+    else
+        launch_kernel(gemm_qkv_kernel<256, C>, dim3(tiles), dim3(C::NT), C::LDS, s, x, w.fh, M, N, K, tiles_n, tiles, e);
+    return hipGetLastError();
+}
+
 hipError_t launch_gemm_qkv(hipStream_t s, const Q8Dev& w, const uint16_t* x, int M, int hd, const QkvEpilogue& e) {
     if (!gemm_operands_ok(w, x, M, e.q) || !gemm_qkv_supported(hd, e.heads, e.kv_heads) || !e.k || (!e.v && !e.vt) ||
         !e.q_norm || !e.k_norm || !e.positions || !e.rope || w.rows != (e.heads + 2 * e.kv_heads) * hd ||
         (e.vt && (!e.vcol || e.vt_cols <= 0)))
         return hipErrorInvalidValue;
     if (M == 0) return hipSuccess;
-    if (e.stage && skinny_ok(w, M)) {
+    if (e.stage && skinny_ok(w, M, 32)) {
         // short batch: the skinny GEMM's fp16 staging, then the row pass (same bits as fused)
         hipError_t r = gemm_skinny_launch<kEpiF16, true, 1>(s, w, x, M, e.stage, e.scale);
         if (r != hipSuccess) return r;
@@ -821,14 +879,11 @@ hipError_t launch_gemm_qkv(hipStream_t s, const Q8Dev& w, const uint16_t* x, int
                           w.rows, e);
         return hipGetLastError();
     }
-    using C = GemmWide;
-    const int N = w.rows, K = w.cols;
-    const int tiles_m = (M + C::BM - 1) / C::BM, tiles_n = (N + C::BN - 1) / C::BN, tiles = tiles_m * tiles_n;
-    if (hd == 128)
-        launch_kernel(gemm_qkv_kernel<128>, dim3(tiles), dim3(C::NT), C::LDS, s, x, w.fh, M, N, K, tiles_n, tiles, e);
-    else
-        launch_kernel(gemm_qkv_kernel<256>, dim3(tiles), dim3(C::NT), C::LDS, s, x, w.fh, M, N, K, tiles_n, tiles, e);
-    return hipGetLastError();
+    // 64-token tiles (one workgroup per CU) while they are at most one per CU, as in launch_gemm_q8.
+    const int64_t halves = int64_t((M + 63) / 64) * ((w.rows + 255) / 256);
+    if (w.cols % GemmQkvHalf::BK == 0 && halves <= g_wide_slots.load(std::memory_order_relaxed) / 2)
+        return gemm_qkv_launch<GemmQkvHalf>(s, w, x, M, hd, e);
+    return gemm_qkv_launch<GemmWide>(s, w, x, M, hd, e);
 }
 
 }  // namespace ge

@@ -60,12 +60,13 @@ struct GemmEpiArgs {
 // K of 32. kEpiGeglu expects W's rows
 // interleaved in 32-row gate/up groups and writes fp16 act[M][N / 2] = gelu_tanh(gate) * up *
 // out_scale. out_scale is a power of two wherever the forward uses it, so it is exact.
-// Batches of at most kSkinnyMaxRows rows (and K a multiple of 128) run on the skinny kernel,
-// one wave per 32-row by 32-column block; the results are bitwise those of the tiled kernel.
-// Up to 512 rows the skinny kernel is the faster of the two at every projection of the
-// config-2 and real-architecture models (at 128 rows 4-6 against 8-18 us; 512 rows is about
-// the crossover), since the tiled kernel's few workgroups sit on a few CUs.
-constexpr int kSkinnyMaxRows = 512;
+// A launch of few rows (K a multiple of 128) runs on the skinny kernel, one wave per 32-row by
+// 32-column block (64 for kEpiGeglu), as long as there are no more waves than CUs; every other one
+// on the tiled kernel, at a tile shape by its size. All give the same bits. Past one wave per CU
+// the skinny kernel loses to small tiles: qkv (1280 x 768) 4.2 against 4.7 us at 192 rows
+// (240 waves), 6.7 against 4.8 at 256 (320); o (768 x 768) 4.2 / 4.7 at 320 rows (240) and
+// 6.6 / 4.9 at 400 (312); gate/up 4.6 / 6.6 at 192 (216) and 7.1 / 6.8 at 256 (288); a 512 x 2048
+// projection 6.8 / 8.6 at 512 (256).
 // kEpiGeluBias and kEpiHeads take their operands from ea (y is then unused by kEpiHeads).
 hipError_t launch_gemm_q8(hipStream_t s, const Q8Dev& w, const uint16_t* x, int M, void* y, GemmEpilogue epi,
                           float out_scale = 1.0f, const GemmEpiArgs* ea = nullptr);
@@ -91,8 +92,8 @@ struct QkvEpilogue {
     int vt_cols = 0;
     int heads = 0;
     int kv_heads = 0;
-    // fp16 scratch of at least M * N halves: lets short batches (M <= kSkinnyMaxRows) take the
-    // skinny GEMM and a separate row pass, with the same results; null = always the fused kernel
+    // fp16 scratch of at least M * N halves: lets short batches take the skinny GEMM and a
+    // separate row pass, with the same results; null = always the fused kernel
     uint16_t* stage = nullptr;
 };
 bool gemm_qkv_supported(int hd, int H, int KV);
