@@ -706,5 +706,18 @@ hipError_t launch_f16_to_f32(hipStream_t s, const uint16_t* src, float* dst, siz
     return hipGetLastError();
 }
 
+// Waits on the constant 100 MHz counter; the iteration count bounds it whatever the counter does
+// (4096 sleeps of 512 cycles, under 2 ms).
+__global__ void spin_kernel(long long ticks) {
+    const long long t0 = wall_clock64();
+    for (int i = 0; i < 4096 && wall_clock64() - t0 < ticks; i++) __builtin_amdgcn_s_sleep(8);
+}
+
+hipError_t launch_spin(hipStream_t s, int us) {
+    if (us < 0 || us > 1000) return hipErrorInvalidValue;
+    launch_kernel(spin_kernel, dim3(1), dim3(64), 0, s, (long long)us * 100);
+    return hipGetLastError();
+}
+
 
 }  // namespace ge

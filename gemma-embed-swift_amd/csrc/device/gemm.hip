@@ -827,8 +827,8 @@ hipError_t launch_gemm_q8(hipStream_t s, const Q8Dev& w, const uint16_t* x, int 
     // Tile shapes by projection and batch rows, from sweeps of the shapes (20 launches back to
     // back, one box). The tile shape does not change the results: every shape runs the same MFMA
     // over the same k order. The 768-wide projections (o, down): 128 x 128 tiles (K in stages of
-    // 64) below 6144 rows, 128 x 256 from 6144 (the config-2 forward's four parts launch them at
-    // 4096 rows each). From 12288 rows the fp16-output projections of at most 1024 outputs whose
+    // 64) below 6144 rows, 128 x 256 from 6144 (the config-2 forward's two parts launch them at
+    // 8192 rows each). From 12288 rows the fp16-output projections of at most 1024 outputs whose
     // width 192 divides (768: o and down) take 256 x 192 tiles: at 16384 rows o 22.6 against
     // 23.2 us (256 x 256), down 30.0 against 31.0. The image tower's 1152-wide o and down stay on
     // 128 x 256 inside the tower: with fp32 outputs 256 x 192 lost (o 72.1 against 63.2 us, down

@@ -232,6 +232,9 @@ hipError_t launch_vit_pool(hipStream_t s, const float* x, const int32_t* row0, c
 hipError_t configure_kernels();
 hipError_t gemm_configure();
 
+// Occupies one wave for about `us` microseconds (at most 1000).
+hipError_t launch_spin(hipStream_t s, int us);
+
 hipError_t launch_f32_to_f16(hipStream_t s, const float* src, uint16_t* dst, size_t n);
 hipError_t launch_f16_to_f32(hipStream_t s, const uint16_t* src, float* dst, size_t n);
 

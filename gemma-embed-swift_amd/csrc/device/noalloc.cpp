@@ -99,9 +99,9 @@ void forward_noalloc(ge_ctx* c, const int32_t* tokens, const int32_t* positions,
     if (!pooled) fail(GE_ERR_INVALID, "null output");
     if (!c->scratch) fail(GE_ERR_STATE, "the no-allocation scratch of device %d is not set up", c->device);
     if (c->prof) fail(GE_ERR_STATE, "the no-allocation forward does not run while profiling is enabled");
-    if (n >= kSplitMinTokens) fail(GE_ERR_INVALID, "the no-allocation forward takes packs below %d tokens", kSplitMinTokens);
-    const BatchPlan b = plan_batch(c, tokens, positions, n, seqs, n_seqs, own_vectors(c), own_vector_rows(c));
-    if (b.n_parts != 1) fail(GE_ERR_STATE, "a pack below %d tokens was split into parts", kSplitMinTokens);
+    if (n >= kNoallocMaxTokens) fail(GE_ERR_INVALID, "the no-allocation forward takes packs below %d tokens", kNoallocMaxTokens);
+    BatchPlan b = plan_batch(c, tokens, positions, n, seqs, n_seqs, own_vectors(c), own_vector_rows(c));
+    b.n_parts = 1;  // one stream (encode); a split plan differs from a whole one only in the order of its work items
     Carver count{nullptr};
     carve(c->model, b, n, n_seqs, count);
     if (count.used > kScratchBytes)

@@ -124,9 +124,11 @@ struct StopPoint {
 // (head dim 512) at 1.1e-2 max relative error against the fp32 oracle.
 constexpr int kPreciseHeadDim = 512;
 
-// Streams a large batch is split over (measured 2, 3, 4: 5.93, 5.93, 5.85 ms at config 2; with
-// 8192-row parts' gate/up launches ending in half tiles, 2 parts 6.18 against 4 parts 6.15 ms).
-constexpr int kMaxParts = 4;
+// Streams a large batch is split over. With tile shapes chosen by each launch's own rows two parts
+// are enough, at half the launches of four: packs of 4096 tokens 2.09 ms on two streams against 2.13 on
+// four (2.30 on one), 8192 3.42 / 3.65 (3.79), 16384 5.80 / 5.94, 32768 11.02 / 11.38 (11.78); the
+// reference's architecture at 4096 tokens 3.28 / 3.72 (3.40), at 8 x 1024 6.70 / 6.64 (6.59).
+constexpr int kMaxParts = 2;
 
 // A short pack's forward captured as a HIP graph, keyed by everything its launches' arguments
 // depend on (see run_graph); exec is null while the shape has been seen only once.
@@ -309,8 +311,12 @@ struct StopPoint;
 void encode(ge_ctx* c, StopPoint* sp);
 // Waits for every stream of the context.
 void drain(ge_ctx* c);
-// Packs of at least this many tokens (of two or more sequences) run as parts on several streams.
-constexpr int kSplitMinTokens = 4096;
+// Packs of at least this many tokens (of two or more sequences) run as parts on several streams:
+// 2048 tokens of 64 1.60 -> 1.45 ms, 3072 1.84 -> 1.69; at 1024 tokens one stream is faster (1.22
+// against 1.32 ms).
+constexpr int kSplitMinTokens = 2048;
+// The no-allocation forward takes packs below this many tokens.
+constexpr int kNoallocMaxTokens = 4096;
 // Takes the device address of the no-allocation forward's scratch array on the context's device
 // (noalloc.cpp); called once per context at creation.
 void noalloc_init(ge_ctx* c);

@@ -28,7 +28,7 @@
 //                             shape. By default on one stream with every launch timed by HIP events
 //                             (ge_profile_enable), so each kernel runs at M = 16384 and the probe
 //                             prints a per-kernel table; with "parts" the pack runs as the timed
-//                             forward does (four parts on four streams, no events)
+//                             forward does (parts on two streams, no events)
 //   ge_probe reference_forward [reps]
 //                             the same for the reference's real architecture (8 x 1024 tokens)
 //   ge_probe calibrate        fp16 -> fp32 conversion of 2^28 values (reads 512 MiB, writes 1 GiB):
@@ -390,7 +390,7 @@ int probe_forward(int reps, bool real_shapes, bool parts) {
     for (float v : out) check += std::fabs(double(v));
     std::printf("%s forward, %d x %d tokens (%s): %.3f ms per forward; sum |pooled| %.6e\n",
                 real_shapes ? "reference shapes" : "config 2", texts, len,
-                parts ? "parts on four streams" : "one stream, every launch timed", ms, check);
+                parts ? "parts on two streams" : "one stream, every launch timed", ms, check);
     if (!parts) {
         std::printf("%-24s %9s %10s %12s\n", "kernel", "launches", "avg us", "ms/forward");
         for (int i = 0;; i++) {

@@ -21,8 +21,8 @@ ROW_SLACK = 256          # kRowSlack, csrc/device/kernels.hpp:29
 ATTN_QUERIES = 32        # kAttnQueries, kernels.hpp:26
 ATTN_QUERIES_V2 = 64     # kAttnQueriesV2, kernels.hpp:139
 SMALL_ITEMS = 256        # kAttnSmallItems, runtime.cpp
-SPLIT_MIN_TOKENS = 4096  # kSplitMinTokens, runtime_internal.hpp
-MAX_PARTS = 4            # kMaxParts, runtime_internal.hpp
+SPLIT_MIN_TOKENS = 2048  # kSplitMinTokens, runtime_internal.hpp
+MAX_PARTS = 2            # kMaxParts, runtime_internal.hpp
 SKINNY_MAX_ROWS = 512    # kSkinnyMaxRows, kernels.hpp
 WORK_BYTES, SEQ_BYTES = 16, 8  # sizeof(AttnWork), sizeof(SeqRange)
 
