@@ -181,10 +181,13 @@ __device__ __forceinline__ int xcd_tile(int b, int tiles) {
 // 4 g + e of acc[i][j] then holds row i * 32 + lane % 32, column j * 32 + g * 8 + (lane / 32) * 4 + e
 // of the wave's block, instead of row i * 32 + g * 8 + (lane / 32) * 4 + e, column j * 32 + lane % 32.
 // Leaves the stage buffers' reads outstanding (the caller waits before reusing LDS).
-template <class C, bool TR>
+// PAIR: W's 32-row blocks alternate between two matrices (gate and up): block j is block
+// (j / 2) * pair_stride of Fh for even j and of Fh2 for odd j.
+template <class C, bool TR, bool PAIR = false>
 __device__ __forceinline__ void gemm_mainloop(const uint16_t* __restrict__ X, const uint16_t* __restrict__ Fh, int M,
                                               int N, int K, int m0, int n0, unsigned char* lds,
-                                              float16_t (&acc)[C::FM][C::FN]) {
+                                              float16_t (&acc)[C::FM][C::FN], const uint16_t* __restrict__ Fh2 = nullptr,
+                                              int pair_stride = 1) {
     using T = DTile<C::BK>;
     constexpr int BK = C::BK, ST = C::ST, KS = C::KS, FM = C::FM, FN = C::FN, AW = C::AW, BW = C::BW;
     constexpr int A_BYTES = C::A_BYTES, STAGE = C::STAGE;
@@ -195,7 +198,12 @@ __device__ __forceinline__ void gemm_mainloop(const uint16_t* __restrict__ X, co
     // Byte offset of this lane's 16 bytes for each of the wave's chunks, at stage 0; a stage
     // adds BK * 2 bytes (activations) or KS KB (weights) through the scalar offset.
     const __amdgpu_buffer_rsrc_t xr = buffer_rsrc(X, uint32_t(M) * uint32_t(K) * 2u);
-    const __amdgpu_buffer_rsrc_t fr = buffer_rsrc(Fh, uint32_t(N) * uint32_t(K) * 2u);
+    // A pair's matrix is chosen once per wave: its weight chunks all lie in one 32-row block.
+    static_assert(!PAIR || KS % BW == 0, "a wave's weight chunks of a stage lie in one 32-row block");
+    const int wave_block = n0 / 32 + __builtin_amdgcn_readfirstlane(wave) * BW / KS;
+    const __amdgpu_buffer_rsrc_t fr =
+        PAIR ? buffer_rsrc(min(wave_block, N / 32 - 1) & 1 ? Fh2 : Fh, uint32_t((N / 64 - 1) * pair_stride + 1) * uint32_t(K) * 64u)
+             : buffer_rsrc(Fh, uint32_t(N) * uint32_t(K) * 2u);
     uint32_t aoff[AW], boff[BW];
 #pragma unroll
     for (int i = 0; i < AW; i++) {
@@ -205,7 +213,7 @@ __device__ __forceinline__ void gemm_mainloop(const uint16_t* __restrict__ X, co
 #pragma unroll
     for (int i = 0; i < BW; i++) {
         const int c = wave * BW + i, jb = c / KS, t = c % KS;
-        const int jg = min(n0 / 32 + jb, N / 32 - 1);
+        const int jn = min(n0 / 32 + jb, N / 32 - 1), jg = PAIR ? jn / 2 * pair_stride : jn;
         boff[i] = uint32_t((((size_t)jg * KT + t) * 512 + lane * 8) * 2);
     }
 #define G_ISSUE(stage, buf)                                                                               \
@@ -307,7 +315,7 @@ __global__ __launch_bounds__(C::NT) void gemm_kernel(const uint16_t* __restrict_
             const int m0 = (tile / tiles_n) * C::BM, n0 = (tile % tiles_n) * C::BN + (hb % 2) * CH::BN;
             if (n0 >= N) return;  // the right half of a last column tile that N ends inside
             float16_t acc[CH::FM][CH::FN];
-            gemm_mainloop<CH, false>(X, Fh, M, N, K, m0, n0, lds, acc);
+            gemm_mainloop<CH, false, EPI == kEpiGeglu>(X, Fh, M, N, K, m0, n0, lds, acc, ea.up, ea.pair_stride);
             gemm_store_tile<CH::FM, CH::FN, EPI>(acc, Y, M, N, m0 + (wave / CH::WN) * CH::TM,
                                                  n0 + (wave % CH::WN) * CH::TN, lane, out_scale, ea);
             return;
@@ -316,7 +324,7 @@ __global__ __launch_bounds__(C::NT) void gemm_kernel(const uint16_t* __restrict_
     const int tile = xcd_tile(blockIdx.x, n_full);
     const int m0 = (tile / tiles_n) * C::BM, n0 = (tile % tiles_n) * C::BN;
     float16_t acc[C::FM][C::FN];
-    gemm_mainloop<C, false>(X, Fh, M, N, K, m0, n0, lds, acc);
+    gemm_mainloop<C, false, EPI == kEpiGeglu>(X, Fh, M, N, K, m0, n0, lds, acc, ea.up, ea.pair_stride);
     gemm_store_tile<C::FM, C::FN, EPI>(acc, Y, M, N, m0 + (wave / C::WN) * C::TM, n0 + (wave % C::WN) * C::TN, lane,
                                        out_scale, ea);
 }
@@ -355,20 +363,24 @@ __global__ __launch_bounds__(64 * kSkinnyWaves) void gemm_skinny_kernel(const ui
     __builtin_assume(KT >= SK);
     asm volatile("" ::"s"(Y), "s"(out_scale));
     const __amdgpu_buffer_rsrc_t xr = buffer_rsrc(X, uint32_t(M) * uint32_t(K) * 2u);
-    const __amdgpu_buffer_rsrc_t fr = buffer_rsrc(Fh, uint32_t(N) * uint32_t(K) * 2u);
+    // a GeGLU pair's column blocks come from two matrices (see gemm_mainloop)
+    constexpr bool PAIR = EPI == kEpiGeglu;
+    static_assert(NJ <= 2 && (!PAIR || NJ == 2), "one gate and one up block");
+    const uint32_t fbytes = PAIR ? uint32_t((N / 64 - 1) * ea.pair_stride + 1) * uint32_t(K) * 64u : uint32_t(N) * uint32_t(K) * 2u;
+    const __amdgpu_buffer_rsrc_t fr[2] = {buffer_rsrc(Fh, fbytes), buffer_rsrc(PAIR ? ea.up : Fh, fbytes)};
     // lane l: activation row rt * 32 + l % 32, k-step columns 8 (l / 32) .. + 8; weight fragment
     // bytes 16 l of the 1 KB chunk (jb, t)
     const uint32_t aoff = uint32_t(((rt * 32 + (lane & 31)) * K + 8 * (lane >> 5)) * 2);
     uint32_t boff[NJ];
 #pragma unroll
-    for (int j = 0; j < NJ; j++) boff[j] = uint32_t(((cg * NJ + j) * KT * 512 + lane * 8) * 2);
+    for (int j = 0; j < NJ; j++) boff[j] = uint32_t(((PAIR ? cg * ea.pair_stride : cg * NJ + j) * KT * 512 + lane * 8) * 2);
     half8_t a[SK], b[SK][NJ];
     // k-step t (wave-uniform) through the scalar offset: no per-load address arithmetic
 #define SK_LOAD(u, t)                                                                                   \
     do {                                                                                                \
         a[u] = __builtin_bit_cast(half8_t, __builtin_amdgcn_raw_buffer_load_b128(xr, aoff, (t) * 32, 0)); \
         _Pragma("unroll") for (int j = 0; j < NJ; j++) b[u][j] =                                        \
-            __builtin_bit_cast(half8_t, __builtin_amdgcn_raw_buffer_load_b128(fr, boff[j], (t) * 1024, 0)); \
+            __builtin_bit_cast(half8_t, __builtin_amdgcn_raw_buffer_load_b128(fr[j], boff[j], (t) * 1024, 0)); \
     } while (0)
     float16_t acc[1][NJ];
 #pragma unroll
@@ -784,7 +796,14 @@ bool skinny_ok(const Q8Dev& w, int M, int cols) {
 
 hipError_t launch_gemm_q8(hipStream_t s, const Q8Dev& w, const uint16_t* x, int M, void* y, GemmEpilogue epi,
                           float out_scale, const GemmEpiArgs* eap) {
-    const GemmEpiArgs ea = eap ? *eap : GemmEpiArgs{};
+    GemmEpiArgs ea = eap ? *eap : GemmEpiArgs{};
+    if (epi == kEpiGeglu) {
+        if (!w.fh) return hipErrorInvalidValue;
+        if (!ea.up) {  // W interleaved: blocks 2 j (gate) and 2 j + 1 (up)
+            ea.up = w.fh + (size_t)w.cols * 32;
+            ea.pair_stride = 2;
+        }
+    }
     if (epi == kEpiHeads) {
         if (!ea.bias || !ea.dst[0] || !ea.dst[1] || !ea.dst[2] || ea.hd <= 0 || ea.hp < ea.hd || ea.heads <= 0 ||
             w.rows != 3 * ea.heads * ea.hd)
@@ -799,7 +818,7 @@ hipError_t launch_gemm_q8(hipStream_t s, const Q8Dev& w, const uint16_t* x, int 
         switch (epi) {
         case kEpiF32: return gemm_skinny_launch<kEpiF32, false, 1>(s, w, x, M, y, out_scale);
         case kEpiF16: return gemm_skinny_launch<kEpiF16, false, 1>(s, w, x, M, y, out_scale);
-        case kEpiGeglu: return gemm_skinny_launch<kEpiGeglu, false, 2>(s, w, x, M, y, out_scale);
+        case kEpiGeglu: return gemm_skinny_launch<kEpiGeglu, false, 2>(s, w, x, M, y, out_scale, ea);
         case kEpiGeluBias: return gemm_skinny_launch<kEpiGeluBias, false, 1>(s, w, x, M, y, out_scale, ea);
         case kEpiHeads: return gemm_skinny_launch<kEpiHeads, false, 1>(s, w, x, M, y, out_scale, ea);
         default: return hipErrorInvalidValue;

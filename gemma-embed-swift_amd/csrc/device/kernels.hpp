@@ -46,7 +46,9 @@ hipError_t launch_q8_fragments(hipStream_t s, const Q8Dev& w, uint16_t* fh);
 
 enum GemmEpilogue { kEpiF32 = 0, kEpiF16 = 1, kEpiGeglu = 2, kEpiGeluBias = 3, kEpiHeads = 4 };
 
-// Operands of the bias epilogues of the image tower. kEpiGeluBias: fp16
+// Operands of the epilogues that need more than the scale. kEpiGeglu: with `up` set, W's fragments
+// (fh) are the gate matrix's alone and `up` the up matrix's (each rows / 2 rows, block stride 1);
+// unset, both come from fh, interleaved. kEpiGeluBias: fp16
 // y[M][N] = gelu_tanh(acc + bias) * out_scale. kEpiHeads: fp16 (acc + bias) * out_scale into three
 // head-padded buffers: column n = (part * heads + head) * hd + e of the product goes to dst[part]
 // at [row][head][e], row stride heads * hp; columns hd .. hp of each head are not written.
@@ -54,6 +56,8 @@ struct GemmEpiArgs {
     const float* bias = nullptr;
     uint16_t* dst[3] = {nullptr, nullptr, nullptr};
     int hd = 0, hp = 0, heads = 0;
+    const uint16_t* up = nullptr;
+    int pair_stride = 1;
 };
 
 // y[M][N] = (x[M][K] (fp16) * W[N][K]^T (Q8_0, through W.fh)) * out_scale; N a multiple of 64,

@@ -35,8 +35,7 @@
 //                             the known-size kernel that scales the HBM byte counters
 //
 // Inputs are synthetic: Q8_0 rows with random int8 quants and fp16 scales, activations uniform
-// in [-0.5, 0.5). Each call of the GeGLU entry point also interleaves the two matrices and builds
-// their fragment-order copy; a profile reads the GEMM kernel's own rows.
+// in [-0.5, 0.5).
 #include <algorithm>
 #include <chrono>
 #include <cmath>
