@@ -14,28 +14,6 @@
 namespace ge {
 namespace {
 
-// Temporary device buffers of one call, freed when it returns.
-struct Temps {
-    std::vector<void*> ptrs;
-    ~Temps() {
-        for (void* p : ptrs) (void)hipFree(p);
-    }
-    template <typename T>
-    T* alloc(size_t count, const char* what) {
-        void* p = dev_alloc(count * sizeof(T), what);
-        ptrs.push_back(p);
-        return static_cast<T*>(p);
-    }
-};
-
-float* device_constant(ge_ctx* c, Temps& t, size_t n, float value) {
-    std::vector<float> h(n, value);
-    float* d = t.alloc<float>(n, "op constant");
-    hip_check(hipMemcpy(d, h.data(), n * 4, hipMemcpyHostToDevice), "upload");
-    (void)c;
-    return d;
-}
-
 template <typename T>
 std::vector<T> read_back(const void* src, size_t n) {
     std::vector<T> h(n);
@@ -43,9 +21,36 @@ std::vector<T> read_back(const void* src, size_t n) {
     return h;
 }
 
+const float* fill_constant(void* p, size_t n, float value) {
+    const std::vector<float> h(n, value);
+    hip_check(hipMemcpy(p, h.data(), n * 4, hipMemcpyHostToDevice), "upload");
+    return static_cast<const float*>(p);
+}
+
 bool row_width_ok(int width) { return width > 0 && width % 4 == 0 && width <= 1024; }
 
 }  // namespace
+
+unsigned char* OpTemps::base() {
+    if (used_ > c_->op_cap) {
+        if (c_->op_buf) hip_check(hipFree(c_->op_buf), "hipFree");
+        c_->op_buf = nullptr;
+        c_->op_cap = 0;
+        c_->op_buf = dev_alloc(used_, "per-op temporaries");
+        c_->op_cap = used_;
+    }
+    return static_cast<unsigned char*>(c_->op_buf);
+}
+
+OpTemps::~OpTemps() {
+    if (c_->op_cap > kOpTempsKept) {
+        (void)hipStreamSynchronize(c_->stream);
+        (void)hipFree(c_->op_buf);
+        c_->op_buf = nullptr;
+        c_->op_cap = 0;
+    }
+}
+
 }  // namespace ge
 
 using ge::fail;
@@ -59,10 +64,12 @@ int ge_op_rmsnorm(ge_ctx* c, const void* x, void* out, const void* w, int32_t ro
         if (!x || !out || rows < 0 || !ge::row_width_ok(width))
             fail(GE_ERR_INVALID, "rmsnorm: rows >= 0 and a width that is a multiple of 4 up to 1024");
         if (rows == 0) return;
-        ge::Temps t;
-        // the forward's standalone norm: out = rmsnorm(x * mul * rscale[row / per_scale]) * w
-        const float* one = ge::device_constant(c, t, 1, 1.0f);
-        const float* wt = w ? static_cast<const float*>(w) : ge::device_constant(c, t, size_t(width), 1.0f);
+        // the forward's standalone norm: out = rmsnorm(x * mul * rscale[row / per_scale]) * w, with
+        // ones for rscale and a missing w
+        ge::OpTemps t(c);
+        const size_t ones = t.reserve(size_t(width) * 4);
+        const float* one = ge::fill_constant(t.base() + ones, w ? 1 : size_t(width), 1.0f);
+        const float* wt = w ? static_cast<const float*>(w) : one;
         ge::launch(c, "rmsnorm", [&] {
             return ge::launch_ple_rmsnorm(c->stream, static_cast<const float*>(x), rows, width, pre_scale, one, rows, wt, eps,
                                           static_cast<float*>(out));
@@ -123,9 +130,10 @@ int ge_op_embed(ge_ctx* c, const ge_q8_matrix* table, const void* tokens, int32_
             if (ids[size_t(i)] < -n_vectors || ids[size_t(i)] >= table->m.rows)
                 fail(GE_ERR_INVALID, "token %d at row %d is neither in the table [0, %d) nor one of the %d vector rows",
                      ids[size_t(i)], i, table->m.rows, n_vectors);
-        ge::Temps t;
-        const float* w = norm_w ? static_cast<const float*>(norm_w) : ge::device_constant(c, t, size_t(d), 1.0f);
-        uint16_t* h = h16 ? static_cast<uint16_t*>(h16) : t.alloc<uint16_t>(size_t(n_tokens) * d, "embed h");
+        ge::OpTemps t(c);
+        const size_t ones = norm_w ? 0 : t.reserve(size_t(d) * 4), rows = h16 ? 0 : t.reserve(size_t(n_tokens) * d * 2);
+        const float* w = norm_w ? static_cast<const float*>(norm_w) : ge::fill_constant(t.base() + ones, size_t(d), 1.0f);
+        uint16_t* h = h16 ? static_cast<uint16_t*>(h16) : reinterpret_cast<uint16_t*>(t.base() + rows);
         ge::launch(c, "embed_norm", [&] {
             return ge::launch_embed_norm(c->stream, table->m, static_cast<const int32_t*>(tokens), n_tokens, scale,
                                          static_cast<const float*>(vectors), w, eps, static_cast<float*>(x), h);

@@ -1578,6 +1578,7 @@ void ge_destroy(ge_ctx* c) {
     ge::free_model(c);
     ge::free_vision(c);
     if (c->vec_buf) (void)hipFree(c->vec_buf);
+    if (c->op_buf) (void)hipFree(c->op_buf);
     for (auto& p : c->prof_pending) {
         (void)hipEventDestroy(p.a);
         (void)hipEventDestroy(p.b);
@@ -1823,18 +1824,7 @@ void op_attention(ge_ctx* c, const void* q, const void* q_lo, const void* k, con
     // The ABI's work items (ge_attention_work) come in; the kernels take ge::AttnWork.
     std::vector<ge_attention_work> items(static_cast<size_t>(n_work), ge_attention_work{});
     hip_check(hipMemcpy(items.data(), work, items.size() * sizeof(ge_attention_work), hipMemcpyDeviceToHost), "read work");
-    std::vector<void*> temps;
-    struct Free {
-        std::vector<void*>* p;
-        ~Free() {
-            for (void* x : *p) (void)hipFree(x);
-        }
-    } guard{&temps};
-    auto temp = [&](size_t bytes) {
-        void* p = dev_alloc(bytes, "attention op");
-        temps.push_back(p);
-        return p;
-    };
+    OpTemps temps(c);
     if (split || attention_v2_supported(head_dim, heads, kv_heads)) {
         // The sequences behind the work items, in order; V transposed into their layout.
         std::vector<ge_seq> seqs;
@@ -1850,9 +1840,12 @@ void op_attention(ge_ctx* c, const void* q, const void* q_lo, const void* k, con
             for (uint32_t q0 = 0; q0 < seqs[s].length; q0 += kAttnQueriesV2)
                 w2.push_back(AttnWork{seqs[s].start, seqs[s].length, q0, vl.start[s]});
         const int kvd = kv_heads * head_dim;
-        auto* vt = static_cast<uint16_t*>(temp(size_t(kvd) * vl.cols * 2));
-        auto* vcol = static_cast<int32_t*>(temp(size_t(T) * 4));
-        auto* dw = static_cast<AttnWork*>(temp(w2.size() * sizeof(AttnWork)));
+        const size_t vt_at = temps.reserve(size_t(kvd) * vl.cols * 2), vcol_at = temps.reserve(size_t(T) * 4),
+                     dw_at = temps.reserve(w2.size() * sizeof(AttnWork));
+        unsigned char* const base = temps.base();
+        auto* vt = reinterpret_cast<uint16_t*>(base + vt_at);
+        auto* vcol = reinterpret_cast<int32_t*>(base + vcol_at);
+        auto* dw = reinterpret_cast<AttnWork*>(base + dw_at);
         hip_check(hipMemsetAsync(vt, 0, size_t(kvd) * vl.cols * 2, c->stream), "hipMemset");
         hip_check(hipMemcpyAsync(vcol, vl.vcol.data(), size_t(T) * 4, hipMemcpyHostToDevice, c->stream), "upload");
         hip_check(hipMemcpyAsync(dw, w2.data(), w2.size() * sizeof(AttnWork), hipMemcpyHostToDevice, c->stream), "upload");
@@ -1872,7 +1865,8 @@ void op_attention(ge_ctx* c, const void* q, const void* q_lo, const void* k, con
     } else {
         std::vector<AttnWork> w1;
         for (const auto& it : items) w1.push_back(AttnWork{it.seq_start, it.seq_len, it.q0, 0});
-        auto* dw = static_cast<AttnWork*>(temp(w1.size() * sizeof(AttnWork)));
+        const size_t dw_at = temps.reserve(w1.size() * sizeof(AttnWork));
+        auto* dw = reinterpret_cast<AttnWork*>(temps.base() + dw_at);
         hip_check(hipMemcpyAsync(dw, w1.data(), w1.size() * sizeof(AttnWork), hipMemcpyHostToDevice, c->stream), "upload");
         launch(c, "attention", [&] {
             return launch_attention(c->stream, static_cast<const uint16_t*>(q), static_cast<const uint16_t*>(k),
