@@ -7,6 +7,7 @@
 // pooling, the projector's weighted RMSNorm and a Q8_0 projection into the text space.
 #include <algorithm>
 #include <cmath>
+#include <cstdlib>
 #include <cstring>
 #include <memory>
 #include <string>
@@ -44,12 +45,17 @@ struct VisionState {
     // staged batch
     int staged_patches = -1, staged_tokens = 0, staged_work = 0;
     int items = kAttnQueriesV2;  // query rows per attention work item of the staged batch
+    // part p: patch rows [part_row[p], part_row[p + 1]) with work items [part_work[p], part_work[p + 1])
+    int n_parts = 1, part_row[kMaxParts + 1] = {0}, part_work[kMaxParts + 1] = {0};
 };
 
 namespace {
 
 // Smallest count of 256-query attention workgroups for which a batch takes them (one per CU).
 constexpr int64_t kVitWideItems = 256;
+
+// Patch rows from which a batch of several images runs as two parts on two streams.
+constexpr int kVitSplitRows = 4096;
 
 VisionState& vision_of(ge_ctx* c) {
     if (!c->vision) fail(GE_ERR_STATE, "no image encoder has been uploaded");
@@ -276,7 +282,7 @@ void ensure_vision_workspace(ge_ctx* c, VisionState& v, int patches, int tokens,
     const int rows = (patches + 63) / 64 * 64 + kRowSlack, tok_rows = (tokens + 63) / 64 * 64 + kRowSlack;
     const bool grow = rows > v.rows || tok_rows > v.tok_rows || work > v.work_cap || vt_cols > v.vt_cap;
     if (!grow) return;
-    hip_check(hipStreamSynchronize(c->stream), "hipStreamSynchronize");
+    drain(c);
     const int r = std::max(rows, v.rows), tr = std::max(tok_rows, v.tok_rows), wc = std::max(std::max(work, 1), v.work_cap);
     const int vc = (std::max(vt_cols, v.vt_cap + v.vt_cap / 2) + 63) / 64 * 64;
     free_vision_workspace(v);
@@ -321,7 +327,9 @@ void alloc_vision_workspace(hipStream_t s, VisionState& v, int r, int tr, int wc
 // VisionBatch.init (VisionTower.swift:17-33) and VisionTower.upload (:113-140): images back to
 // back as patch rows (patch i of an image at column i % gx, row i / gx), each image one attention
 // sequence, pooled tokens back to back in (oy, ox) order.
-void vision_stage(ge_ctx* c, const float* patches, int n_patches, const ge_image_grid* grids, int n_images) {
+// upload false: the patches stay with the caller, who gives them to vision_encode.
+void vision_stage(ge_ctx* c, const float* patches, int n_patches, const ge_image_grid* grids, int n_images,
+                  bool upload = true) {
     VisionState& v = vision_of(c);
     if (n_images <= 0 || !grids) fail(GE_ERR_INVALID, "a batch needs at least one image");
     if (!patches) fail(GE_ERR_INVALID, "null patches");
@@ -367,20 +375,32 @@ void vision_stage(ge_ctx* c, const float* patches, int n_patches, const ge_image
         const void* src;
         size_t bytes;
     };
-    const Piece pieces[] = {{v.patches32, patches, size_t(n_patches) * v.area * 4},
+    const Piece pieces[] = {{v.patches32, patches, upload ? size_t(n_patches) * v.area * 4 : 0},
                             {v.px, px.data(), px.size() * 4},
                             {v.py, py.data(), py.size() * 4},
                             {v.vcol, vcol.data(), vcol.size() * 4},
                             {v.tok_row0, row0.data(), row0.size() * 4},
                             {v.tok_gx, gxs.data(), gxs.size() * 4},
                             {v.work, work.data(), work.size() * sizeof(AttnWork)}};
-    hip_check(hipStreamSynchronize(c->stream), "hipStreamSynchronize");
+    drain(c);
     for (const Piece& pc : pieces)
         if (pc.bytes) hip_check(hipMemcpy(pc.dst, pc.src, pc.bytes, hipMemcpyHostToDevice), "upload image batch");
     v.staged_patches = n_patches;
     v.staged_tokens = tokens;
     v.staged_work = int(work.size());
     v.items = items;
+    // Two parts of whole images, cut at the image start nearest to the middle.
+    int cut = 0;
+    if (n_patches >= kVitSplitRows)
+        for (const AttnWork& a : work)
+            if (std::abs(2 * int(a.seq_start) - n_patches) < std::abs(2 * cut - n_patches)) cut = int(a.seq_start);
+    v.n_parts = cut > 0 ? 2 : 1;
+    v.part_row[1] = cut > 0 ? cut : n_patches;
+    v.part_row[2] = n_patches;
+    v.part_work[1] = int(std::lower_bound(work.begin(), work.end(), uint32_t(v.part_row[1]),
+                                          [](const AttnWork& a, uint32_t row) { return a.seq_start < row; }) -
+                         work.begin());
+    v.part_work[2] = int(work.size());
 }
 
 // ---------------------------------------------------------------- forward
@@ -396,21 +416,40 @@ struct VitStop {
     }
 };
 
+// The encoder's layers over one part of the staged batch: patch rows [r0, r0 + P) and their work
+// items, on one stream. Parts run beside each other, unsynchronised: every buffer's rows (and V^T's
+// columns) are a part's own, at the same place in every layer. The attention kernels index absolute
+// rows, so they take the buffers' bases.
+struct VitPart {
+    hipStream_t s;
+    int r0, P;
+    const AttnWork* work;
+    int n_work;
+};
+
 // VisionTower.encode (VisionTower.swift:143-185) for config 5's encoder: 8 launches per layer.
-void vision_encode(ge_ctx* c, VitStop* sp) {
+// Returns true when it stopped at the traced tensor.
+bool vision_layers(ge_ctx* c, const VitPart& p, VitStop* sp) {
     VisionState& v = vision_of(c);
-    if (v.staged_patches < 0) fail(GE_ERR_STATE, "no image batch is staged");
-    const int P = v.staged_patches, T = v.staged_tokens, D = v.hidden;
-    hipStream_t s = c->stream;
+    const int P = p.P, D = v.hidden, HP = v.heads * v.hp;
+    hipStream_t s = p.s;
+    auto rows = [&](auto* base, int width) { return base + size_t(p.r0) * width; };
     auto stop = [&](const char* n, int l) { return sp && sp->at(n, l); };
-    launch(c, "vit_patches_f16", [&] { return launch_f32_to_f16(s, v.patches32, v.patches16, size_t(P) * v.area); });
-    launch(c, "vit_gemm_patch", [&] { return launch_gemm_q8(s, v.patch_w, v.patches16, P, v.t, kEpiF32); });
-    if (stop("inp", -1)) return;
-    launch(c, "vit_embed", [&] {
-        return launch_vit_embed(s, v.t, v.patch_b, v.pos, v.npos, v.px, v.py, P, D, v.layer[0].ln1_w, v.layer[0].ln1_b,
-                                v.eps, v.x, v.h);
+    float* const x = rows(v.x, D);
+    float* const t = rows(v.t, D);
+    uint16_t* const h = rows(v.h, D);
+    uint16_t* const o16 = rows(v.o16, D);
+    uint16_t* const act = rows(v.act, v.ff_pad);
+    launch(c, "vit_patches_f16", [&] {
+        return launch_f32_to_f16(s, rows(v.patches32, v.area), rows(v.patches16, v.area), size_t(P) * v.area);
     });
-    if (stop("pos_embd", -1) || stop("layer_inp_normed", 0)) return;
+    launch(c, "vit_gemm_patch", [&] { return launch_gemm_q8(s, v.patch_w, rows(v.patches16, v.area), P, t, kEpiF32); });
+    if (stop("inp", -1)) return true;
+    launch(c, "vit_embed", [&] {
+        return launch_vit_embed(s, t, v.patch_b, v.pos, v.npos, v.px + p.r0, v.py + p.r0, P, D, v.layer[0].ln1_w,
+                                v.layer[0].ln1_b, v.eps, x, h);
+    });
+    if (stop("pos_embd", -1) || stop("layer_inp_normed", 0)) return true;
     // softmax(q k^T / sqrt(hd)); q and k arrive multiplied by qkv_c
     const float att_scale = 1.0f / std::sqrt(float(v.hd));
     for (int l = 0; l < v.layers; l++) {
@@ -418,53 +457,97 @@ void vision_encode(ge_ctx* c, VitStop* sp) {
         launch(c, "vit_gemm_qkv", [&] {
             GemmEpiArgs ea;
             ea.bias = L.bqkv;
-            ea.dst[0] = v.q;
-            ea.dst[1] = v.k;
-            ea.dst[2] = v.v;
+            ea.dst[0] = rows(v.q, HP);
+            ea.dst[1] = rows(v.k, HP);
+            ea.dst[2] = rows(v.v, HP);
             ea.hd = v.hd;
             ea.hp = v.hp;
             ea.heads = v.heads;
-            return launch_gemm_q8(s, L.wqkv, v.h, P, nullptr, kEpiHeads, L.qkv_c, &ea);
+            return launch_gemm_q8(s, L.wqkv, h, P, nullptr, kEpiHeads, L.qkv_c, &ea);
         });
-        if (stop("Qcur", l) || stop("Kcur", l) || stop("Vcur", l)) return;
-        launch(c, "v_transpose", [&] { return launch_v_transpose(s, v.v, P, v.heads * v.hp, v.vcol, v.vt_cap, v.vt); });
+        if (stop("Qcur", l) || stop("Kcur", l) || stop("Vcur", l)) return true;
+        launch(c, "v_transpose", [&] { return launch_v_transpose(s, rows(v.v, HP), P, HP, v.vcol + p.r0, v.vt_cap, v.vt); });
         launch(c, "vit_attention", [&] {
             const float sc = att_scale / (L.qkv_c * L.qkv_c);
             if (v.hp != v.hd)
-                return launch_attention_padded(s, v.q, v.k, v.vt, v.vt_cap, v.attn, v.work, v.staged_work, v.heads, v.heads,
-                                               v.hp, v.hd, 0, sc, v.items);
-            return launch_attention_v2(s, v.q, v.k, v.vt, v.vt_cap, v.attn, v.work, v.staged_work, v.heads, v.heads, v.hd, 0,
-                                       sc);
+                return launch_attention_padded(s, v.q, v.k, v.vt, v.vt_cap, v.attn, p.work, p.n_work, v.heads, v.heads, v.hp,
+                                               v.hd, 0, sc, v.items);
+            return launch_attention_v2(s, v.q, v.k, v.vt, v.vt_cap, v.attn, p.work, p.n_work, v.heads, v.heads, v.hd, 0, sc);
         });
-        if (stop("kqv_out", l)) return;
+        if (stop("kqv_out", l)) return true;
         // The attention output in fp16 (times o_c). x is stored once per layer: the attention
         // residual's launch writes only the MLP input h (and x only when a trace wants the sum after
         // attention), and the MLP residual's launch recomputes that sum beside its own.
-        launch(c, "vit_gemm_o", [&] { return launch_gemm_q8(s, L.wo, v.attn, P, v.o16, kEpiF16, L.o_c / L.qkv_c); });
-        if (stop("attn_out", l)) return;
+        launch(c, "vit_gemm_o", [&] {
+            return launch_gemm_q8(s, L.wo, rows(v.attn, v.heads * v.hd), P, o16, kEpiF16, L.o_c / L.qkv_c);
+        });
+        if (stop("attn_out", l)) return true;
         const bool store_sum = sp && !sp->hit && sp->layer == l && sp->name == "ffn_inp";
         launch(c, "vit_residual_ln_h", [&] {
-            return launch_vit_residual2_ln(s, store_sum ? 1 : 0, v.x, v.o16, 1.0f / L.o_c, L.bo, nullptr, 1.0f, nullptr,
-                                           L.ln2_w, L.ln2_b, v.eps, P, D, v.h);
+            return launch_vit_residual2_ln(s, store_sum ? 1 : 0, x, o16, 1.0f / L.o_c, L.bo, nullptr, 1.0f, nullptr, L.ln2_w,
+                                           L.ln2_b, v.eps, P, D, h);
         });
-        if (stop("ffn_inp", l) || stop("ffn_inp_normed", l)) return;
+        if (stop("ffn_inp", l) || stop("ffn_inp_normed", l)) return true;
         launch(c, "vit_gemm_up", [&] {
             GemmEpiArgs ea;
             ea.bias = L.bup;
-            return launch_gemm_q8(s, L.wup, v.h, P, v.act, kEpiGeluBias, L.act_c, &ea);
+            return launch_gemm_q8(s, L.wup, h, P, act, kEpiGeluBias, L.act_c, &ea);
         });
-        if (stop("ffn_gelu", l)) return;
-        // the down projection in fp16 (times down_c) over the start of t
-        uint16_t* const d16 = reinterpret_cast<uint16_t*>(v.t);
-        launch(c, "vit_gemm_down", [&] { return launch_gemm_q8(s, L.wdown, v.act, P, d16, kEpiF16, L.down_c / L.act_c); });
-        if (stop("ffn_out", l)) return;
+        if (stop("ffn_gelu", l)) return true;
+        // the down projection in fp16 (times down_c) over the start of the part's rows of t
+        uint16_t* const d16 = reinterpret_cast<uint16_t*>(t);
+        launch(c, "vit_gemm_down", [&] { return launch_gemm_q8(s, L.wdown, act, P, d16, kEpiF16, L.down_c / L.act_c); });
+        if (stop("ffn_out", l)) return true;
         const bool last = l + 1 == v.layers;
         launch(c, "vit_residual_ln_two", [&] {
             const VitLayer* N = last ? nullptr : &v.layer[size_t(l) + 1];
-            return launch_vit_residual2_ln(s, 2, v.x, v.o16, 1.0f / L.o_c, L.bo, d16, 1.0f / L.down_c, L.bdown,
-                                           N ? N->ln1_w : nullptr, N ? N->ln1_b : nullptr, v.eps, P, D, v.h);
+            return launch_vit_residual2_ln(s, 2, x, o16, 1.0f / L.o_c, L.bo, d16, 1.0f / L.down_c, L.bdown,
+                                           N ? N->ln1_w : nullptr, N ? N->ln1_b : nullptr, v.eps, P, D, h);
         });
-        if (stop("layer_out", l) || stop("layer_inp_normed", l + 1)) return;
+        if (stop("layer_out", l) || stop("layer_inp_normed", l + 1)) return true;
+    }
+    return false;
+}
+
+// The tower over the staged batch. A batch of several images and kVitSplitRows patch rows or more
+// runs as two parts on the context's two streams: one part's memory-bound passes and kernel tails
+// overlap the other's work. host_patches: the batch's patches, still with the caller: each part's
+// are copied ahead of its own layers, the second part's while the first one runs; ev_start is
+// recorded after the first copy, so a call's GPU seconds start where the tower does. The caller
+// synchronises before it gives the memory back. Traced and profiled forwards run as one part.
+void vision_encode(ge_ctx* c, VitStop* sp, const float* host_patches = nullptr) {
+    VisionState& v = vision_of(c);
+    if (v.staged_patches < 0) fail(GE_ERR_STATE, "no image batch is staged");
+    const int T = v.staged_tokens, D = v.hidden;
+    hipStream_t s = c->stream;
+    auto stop = [&](const char* n, int l) { return sp && sp->at(n, l); };
+    auto copy_patches = [&](hipStream_t to, int r0, int r1) {
+        if (!host_patches) return;
+        hip_check(hipMemcpyAsync(v.patches32 + size_t(r0) * v.area, host_patches + size_t(r0) * v.area,
+                                 size_t(r1 - r0) * v.area * 4, hipMemcpyHostToDevice, to), "upload patches");
+        if (r0 == 0) hip_check(hipEventRecord(c->ev_start, to), "hipEventRecord");
+    };
+    if (v.n_parts == 1 || sp || c->prof) {
+        copy_patches(s, 0, v.staged_patches);
+        if (vision_layers(c, VitPart{s, 0, v.staged_patches, v.work, v.staged_work}, sp)) return;
+    } else {
+        hipStream_t s2 = c->part_stream[1];
+        hip_check(hipEventRecord(c->ev_fork, s), "hipEventRecord");
+        hip_check(hipStreamWaitEvent(s2, c->ev_fork, 0), "hipStreamWaitEvent");
+        try {
+            for (int i = 0; i < 2; i++) {
+                const VitPart p{i ? s2 : s, v.part_row[i], v.part_row[i + 1] - v.part_row[i], v.work + v.part_work[i],
+                                v.part_work[i + 1] - v.part_work[i]};
+                copy_patches(p.s, p.r0, p.r0 + p.P);
+                vision_layers(c, p, nullptr);
+            }
+        } catch (...) {
+            (void)hipStreamSynchronize(s);
+            (void)hipStreamSynchronize(s2);
+            throw;
+        }
+        hip_check(hipEventRecord(c->part_join[1], s2), "hipEventRecord");
+        hip_check(hipStreamWaitEvent(s, c->part_join[1], 0), "hipStreamWaitEvent");
     }
     launch(c, "vit_pool", [&] {
         return launch_vit_pool(s, v.x, v.tok_row0, v.tok_gx, T, v.merge, D, v.post_w, v.post_b, v.eps, v.norm_w, v.pooled,
@@ -657,9 +740,8 @@ int ge_vision_encode(ge_ctx* c, const float* patches, int32_t n_patches, const g
                      float* vectors, size_t vectors_count, double* gpu_seconds) {
     if (!vectors) return GE_ERR_INVALID;
     return ge::guarded(c, [&] {
-        ge::vision_stage(c, patches, n_patches, grids, n_images);
-        ge::hip_check(hipEventRecord(c->ev_start, c->stream), "hipEventRecord");
-        ge::vision_encode(c, nullptr);
+        ge::vision_stage(c, patches, n_patches, grids, n_images, false);
+        ge::vision_encode(c, nullptr, patches);
         ge::hip_check(hipEventRecord(c->ev_stop, c->stream), "hipEventRecord");
         if (gpu_seconds) {
             ge::hip_check(hipEventSynchronize(c->ev_stop), "hipEventSynchronize");
