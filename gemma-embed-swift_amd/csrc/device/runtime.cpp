@@ -1835,9 +1835,14 @@ void op_attention(ge_ctx* c, const void* q, const void* q_lo, const void* k, con
             T = std::max(T, int(it.seq_start + it.seq_len));
         }
         const VtLayout vl = vt_layout(T, seqs.data(), int(seqs.size()));
+        // 32-query items where the forward takes them (plan_batch): for 9 texts of 130 to 997 tokens
+        // (93 items of 64) the kernel takes 29.7 us against 37.8
+        int64_t items64 = 0;
+        for (const ge_seq& q : seqs) items64 += (int64_t(q.length) + kAttnQueriesV2 - 1) / kAttnQueriesV2;
+        const int item_queries = !split && heads / kv_heads <= 3 && items64 * kv_heads < kAttnSmallItems ? 32 : kAttnQueriesV2;
         std::vector<AttnWork> w2;
         for (size_t s = 0; s < seqs.size(); s++)
-            for (uint32_t q0 = 0; q0 < seqs[s].length; q0 += kAttnQueriesV2)
+            for (uint32_t q0 = 0; q0 < seqs[s].length; q0 += uint32_t(item_queries))
                 w2.push_back(AttnWork{seqs[s].start, seqs[s].length, q0, vl.start[s]});
         const int kvd = kv_heads * head_dim;
         const size_t vt_at = temps.reserve(size_t(kvd) * vl.cols * 2), vcol_at = temps.reserve(size_t(T) * 4),
@@ -1860,7 +1865,7 @@ void op_attention(ge_ctx* c, const void* q, const void* q_lo, const void* k, con
                                               static_cast<const uint16_t*>(k_lo), vt, vl.cols, static_cast<uint16_t*>(out), dw,
                                               int(w2.size()), heads, kv_heads, head_dim, half_window, scale, kAttnQueriesV2);
             return launch_attention_v2(c->stream, qh, kh, vt, vl.cols, static_cast<uint16_t*>(out), dw, int(w2.size()), heads,
-                                       kv_heads, head_dim, half_window, scale);
+                                       kv_heads, head_dim, half_window, scale, item_queries);
         });
     } else {
         std::vector<AttnWork> w1;
