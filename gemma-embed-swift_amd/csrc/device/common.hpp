@@ -35,10 +35,28 @@ typedef float float16_t __attribute__((ext_vector_type(16)));
 // registers.
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 
-__device__ __forceinline__ float wave_sum(float v) {
-#pragma unroll
-    for (int m = 32; m >= 1; m >>= 1) v += __shfl_xor(v, m, 64);
+// The sum over the wave's lanes, the butterfly over xor 32, 16, 8, 4, 2, 1 in VALU lane moves instead of
+// LDS shuffles (about 100 cycles each, a chain of six): the gfx950 half and row swaps, then DPP moves.
+// A rotation by 8 within a row of 16 is xor 8; after it the values repeat every 8 lanes, so a rotation
+// by 4 brings xor 4's. Addition commutes, so the bits are those of the shuffles. A 12-token forward of
+// config 2's model 769 -> 754 us, of the reference's architecture 1217 -> 1175 us.
+template <int CTRL>
+__device__ __forceinline__ float dpp_move(float v) {
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xf, 0xf, true));
+}
+// The last four steps: the sum over each row of 16 lanes.
+__device__ __forceinline__ float row16_sum(float v) {
+    v += dpp_move<0x128>(v);  // row_ror:8
+    v += dpp_move<0x124>(v);  // row_ror:4
+    v += dpp_move<0x4e>(v);   // quad_perm 2, 3, 0, 1
+    v += dpp_move<0xb1>(v);   // quad_perm 1, 0, 3, 2
     return v;
+}
+__device__ __forceinline__ float wave_sum(float v) {
+    const auto a = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    v = __uint_as_float(a[0]) + __uint_as_float(a[1]);
+    const auto b = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return row16_sum(__uint_as_float(b[0]) + __uint_as_float(b[1]));
 }
 
 __device__ __forceinline__ float gelu_tanh(float x) {

@@ -463,8 +463,12 @@ __device__ __forceinline__ void qkv_unit(const half8_t x0, const half8_t x1, con
         f1[e] = float(x1[e]);
         ss = __builtin_fmaf(f1[e], f1[e], __builtin_fmaf(f0[e], f0[e], ss));
     }
+    if constexpr (LPR == 16) {
+        ss = row16_sum(ss);
+    } else {
 #pragma unroll
-    for (int m = LPR / 2; m >= 1; m >>= 1) ss += __shfl_xor(ss, m, 64);
+        for (int m = LPR / 2; m >= 1; m >>= 1) ss += __shfl_xor(ss, m, 64);
+    }
     const float inv = 1.0f / sqrtf(ss / float(HD) + eps);
     if (rope) {
         const float4_t w00 = *reinterpret_cast<const float4_t*>(wnorm + k8);
