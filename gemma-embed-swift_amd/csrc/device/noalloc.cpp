@@ -83,11 +83,9 @@ Workspace carve(const DevModel& m, const BatchPlan& b, int n, int n_seqs, Carver
     w.pooled = cv.take<float>(size_t(n_seqs) * m.out_dims);
     w.pooled_n = cv.take<float>(size_t(n_seqs) * m.hidden);
     // the producer-wave attention's work list, read only by layers off the LDS-copy attention
-    w.work_cap = m.all_v2 ? 0 : std::max(int(b.work.size()), 1);
-    w.work = m.all_v2 ? nullptr : cv.take<AttnWork>(size_t(w.work_cap));
+    w.work = m.all_v2 ? nullptr : cv.take<AttnWork>(std::max(b.work.size(), size_t(1)));
     if (m.any_v2) {
-        w.work2_cap = std::max(int(b.work2.size()), 1);
-        w.work2 = cv.take<AttnWork>(size_t(w.work2_cap));
+        w.work2 = cv.take<AttnWork>(std::max(b.work2.size(), size_t(1)));
         w.vt_cap = (b.vl.cols + 63) / 64 * 64;
         w.vt = cv.take<uint16_t>(size_t(m.max_kvd) * w.vt_cap);
     }

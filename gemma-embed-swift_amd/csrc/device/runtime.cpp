@@ -444,8 +444,8 @@ void free_model(ge_ctx* c) {
 void free_workspace(ge_ctx* c) {
     drop_graphs(c);
     Workspace& w = c->ws;
-    void* ps[] = {w.x, w.qkv, w.t, w.out, w.h, w.q, w.k, w.v, w.attn, w.act, w.tokens, w.positions, w.seqs, w.work, w.pooled,
-                  w.vt, w.vcol, w.work2, w.ple, w.ple_t, w.rs, w.rs2, w.x16, w.g16, w.h3, w.q_lo, w.k_lo, w.hn,
+    void* ps[] = {w.x, w.qkv, w.t, w.out, w.h, w.q, w.k, w.v, w.attn, w.act, w.in, w.pooled,
+                  w.vt, w.ple, w.ple_t, w.rs, w.rs2, w.x16, w.g16, w.h3, w.q_lo, w.k_lo, w.hn,
                   w.pooled_n};
     for (void* p : ps)
         if (p) (void)hipFree(p);
@@ -600,39 +600,39 @@ T* ws_alloc(hipStream_t s, size_t rows, size_t width, const char* what) {
     return static_cast<T*>(p);
 }
 
-// Whether ensure_workspace would reallocate any buffer for a batch of this size.
-bool workspace_grows(const ge_ctx* c, int tokens, int seqs, int work, int work2, int vt_cols) {
+// Whether ensure_workspace would reallocate any buffer for a batch of this size (in_bytes: of its small
+// arrays).
+bool workspace_grows(const ge_ctx* c, int tokens, int seqs, size_t in_bytes, int vt_cols) {
     const Workspace& w = c->ws;
     const DevModel& m = c->model;
     const int rows = (tokens + 63) / 64 * 64 + kRowSlack;
-    return rows > w.rows || seqs > w.seq_cap || !w.seqs || work > w.work_cap || !w.work ||
-           (m.any_v2 && (work2 > w.work2_cap || !w.work2 || vt_cols > w.vt_cap || !w.vt));
+    return rows > w.rows || seqs > w.seq_cap || !w.pooled || in_bytes > w.in_cap || !w.in ||
+           (m.any_v2 && (vt_cols > w.vt_cap || !w.vt));
 }
 
-void ensure_workspace_impl(ge_ctx* c, int tokens, int seqs, int work, int work2, int vt_cols);
+void ensure_workspace_impl(ge_ctx* c, int tokens, int seqs, size_t in_bytes, int vt_cols);
 
 // Grows the workspace for a batch. If an allocation fails, the whole workspace is freed before
 // the error propagates, so no capacity is ever recorded for a buffer that does not exist.
-void ensure_workspace(ge_ctx* c, int tokens, int seqs, int work, int work2, int vt_cols) {
-    if (!workspace_grows(c, tokens, seqs, work, work2, vt_cols)) return;
+void ensure_workspace(ge_ctx* c, int tokens, int seqs, size_t in_bytes, int vt_cols) {
+    if (!workspace_grows(c, tokens, seqs, in_bytes, vt_cols)) return;
     drop_graphs(c);
     try {
-        ensure_workspace_impl(c, tokens, seqs, work, work2, vt_cols);
+        ensure_workspace_impl(c, tokens, seqs, in_bytes, vt_cols);
     } catch (...) {
         free_workspace(c);
         throw;
     }
 }
 
-void ensure_workspace_impl(ge_ctx* c, int tokens, int seqs, int work, int work2, int vt_cols) {
+void ensure_workspace_impl(ge_ctx* c, int tokens, int seqs, size_t in_bytes, int vt_cols) {
     Workspace& w = c->ws;
     const DevModel& m = c->model;
     const int rows = (tokens + 63) / 64 * 64 + kRowSlack;
     if (rows > w.rows) {
-        const int keep_seq = w.seq_cap, keep_work = w.work_cap;
+        const int keep_seq = w.seq_cap;
         free_workspace(c);
         w.seq_cap = keep_seq;
-        w.work_cap = keep_work;
         w.rows = rows;
         w.x = ws_alloc<float>(c->stream, rows, m.hidden, "x");
         w.h = ws_alloc<uint16_t>(c->stream, rows, m.hidden, "h");
@@ -645,9 +645,6 @@ void ensure_workspace_impl(ge_ctx* c, int tokens, int seqs, int work, int work2,
         w.act = ws_alloc<uint16_t>(c->stream, rows, m.ff, "act");
         w.out = ws_alloc<float>(c->stream, rows, m.out_dims, "out");
         w.hn = ws_alloc<float>(c->stream, rows, m.hidden, "final norm");
-        w.tokens = ws_alloc<int32_t>(c->stream, rows, 1, "tokens");
-        w.positions = ws_alloc<int32_t>(c->stream, rows, 1, "positions");
-        w.vcol = ws_alloc<int32_t>(c->stream, rows, 1, "vt columns");
         if (m.any_precise) {
             w.h3 = ws_alloc<uint16_t>(c->stream, rows, 3 * size_t(m.hidden), "split-precision input");
             w.q_lo = ws_alloc<uint16_t>(c->stream, rows, m.max_qd, "q low halves");
@@ -661,37 +658,28 @@ void ensure_workspace_impl(ge_ctx* c, int tokens, int seqs, int work, int work2,
             w.x16 = ws_alloc<uint16_t>(c->stream, rows, m.hidden, "scaled residual");
             w.g16 = ws_alloc<uint16_t>(c->stream, rows, m.pl, "per-layer gate");
         }
-        w.seqs = nullptr;
-        w.work = nullptr;
+        w.in = nullptr;
+        w.in_cap = 0;
         w.pooled = nullptr;
         w.pooled_n = nullptr;
         w.seq_cap = 0;
-        w.work_cap = 0;
         w.vt = nullptr;
-        w.work2 = nullptr;
         w.vt_cap = 0;
-        w.work2_cap = 0;
     }
-    if (seqs > w.seq_cap || !w.seqs) {
-        if (w.seqs) (void)hipFree(w.seqs);
+    if (seqs > w.seq_cap || !w.pooled) {
         if (w.pooled) (void)hipFree(w.pooled);
         if (w.pooled_n) (void)hipFree(w.pooled_n);
-        w.seqs = nullptr;
         w.pooled = w.pooled_n = nullptr;
         w.seq_cap = std::max(seqs, 1);
-        w.seqs = ws_alloc<SeqRange>(c->stream, w.seq_cap, 1, "sequences");
         w.pooled = ws_alloc<float>(c->stream, w.seq_cap, m.out_dims, "pooled");
         w.pooled_n = ws_alloc<float>(c->stream, w.seq_cap, m.hidden, "pooled rows");
     }
-    if (work > w.work_cap || !w.work) {
-        if (w.work) (void)hipFree(w.work);
-        w.work_cap = std::max(work, 1);
-        w.work = ws_alloc<AttnWork>(c->stream, w.work_cap, 1, "attention work");
-    }
-    if (m.any_v2 && (work2 > w.work2_cap || !w.work2)) {
-        if (w.work2) (void)hipFree(w.work2);
-        w.work2_cap = std::max(work2, 1);
-        w.work2 = ws_alloc<AttnWork>(c->stream, w.work2_cap, 1, "attention work");
+    if (in_bytes > w.in_cap || !w.in) {
+        if (w.in) (void)hipFree(w.in);
+        w.in = nullptr;
+        // room for packs a little longer or of more sequences than this one
+        w.in_cap = in_bytes + in_bytes / 4 + 4096;
+        w.in = ws_alloc<unsigned char>(c->stream, w.in_cap, 1, "staged batch");
     }
     // Zero-filled once: columns no token writes (alignment gaps, slack) stay finite, and keys
     // read from them are masked, so they contribute exact zeros.
@@ -835,25 +823,35 @@ void set_staged(ge_ctx* c, const BatchPlan& b, int n, int n_seqs, const float* v
 void stage(ge_ctx* c, const int32_t* tokens, const int32_t* positions, int n, const ge_seq* seqs, int n_seqs,
            const float* vectors, int n_vectors) {
     const BatchPlan b = plan_batch(c, tokens, positions, n, seqs, n_seqs, vectors, n_vectors);
-    // The workspace may be reallocated below: nothing queued may still use it.
-    if (workspace_grows(c, n, n_seqs, int(b.work.size()), int(b.work2.size()), b.vl.cols)) drain(c);
-    ensure_workspace(c, n, n_seqs, int(b.work.size()), int(b.work2.size()), b.vl.cols);
-    Workspace& w = c->ws;
-    // The small arrays go through one pinned buffer: asynchronous copies, no wait for them here
-    // (the forward's kernels follow them on the same stream).
+    // The small arrays, one after another in one pinned buffer and one device block: an asynchronous
+    // copy, no wait for it here (the forward's kernels follow it on the same stream).
     struct Piece {
-        void* dst;
         const void* src;
-        size_t bytes;
+        size_t bytes, at;
     };
-    const Piece pieces[] = {{w.tokens, tokens, size_t(n) * 4},
-                            {w.positions, positions, size_t(n) * 4},
-                            {w.seqs, b.sr.data(), b.sr.size() * sizeof(SeqRange)},
-                            {w.work, b.work.data(), b.work.size() * sizeof(AttnWork)},
-                            {w.work2, b.work2.data(), b.work2.size() * sizeof(AttnWork)},
-                            {w.vcol, b.vl.vcol.data(), b.work2.empty() ? 0 : size_t(n) * 4}};
+    const DevModel& m = c->model;
+    Piece pieces[] = {{tokens, size_t(n) * 4, 0},
+                      {positions, size_t(n) * 4, 0},
+                      {b.sr.data(), b.sr.size() * sizeof(SeqRange), 0},
+                      // read only by layers off the LDS-copy attention
+                      {b.work.data(), m.all_v2 ? 0 : b.work.size() * sizeof(AttnWork), 0},
+                      {b.work2.data(), b.work2.size() * sizeof(AttnWork), 0},
+                      {b.vl.vcol.data(), b.work2.empty() ? 0 : size_t(n) * 4, 0}};
     size_t total = 0;
-    for (const Piece& pc : pieces) total += (pc.bytes + 255) / 256 * 256;
+    for (Piece& pc : pieces) {
+        pc.at = total;
+        total += (pc.bytes + 255) / 256 * 256;
+    }
+    // The workspace may be reallocated below: nothing queued may still use it.
+    if (workspace_grows(c, n, n_seqs, total, b.vl.cols)) drain(c);
+    ensure_workspace(c, n, n_seqs, total, b.vl.cols);
+    Workspace& w = c->ws;
+    w.tokens = reinterpret_cast<int32_t*>(w.in + pieces[0].at);
+    w.positions = reinterpret_cast<int32_t*>(w.in + pieces[1].at);
+    w.seqs = reinterpret_cast<SeqRange*>(w.in + pieces[2].at);
+    w.work = reinterpret_cast<AttnWork*>(w.in + pieces[3].at);
+    w.work2 = reinterpret_cast<AttnWork*>(w.in + pieces[4].at);
+    w.vcol = reinterpret_cast<int32_t*>(w.in + pieces[5].at);
     if (c->staged_copy_recorded) hip_check(hipEventSynchronize(c->staged_copy), "hipEventSynchronize");
     if (total > c->pinned_cap) {
         if (c->pinned) hip_check(hipHostFree(c->pinned), "hipHostFree");
@@ -863,14 +861,9 @@ void stage(ge_ctx* c, const int32_t* tokens, const int32_t* positions, int n, co
         hip_check(hipHostMalloc(&c->pinned, cap, hipHostMallocDefault), "hipHostMalloc");
         c->pinned_cap = cap;
     }
-    size_t off = 0;
-    for (const Piece& pc : pieces) {
-        if (pc.bytes == 0) continue;
-        unsigned char* h = static_cast<unsigned char*>(c->pinned) + off;
-        std::memcpy(h, pc.src, pc.bytes);
-        hip_check(hipMemcpyAsync(pc.dst, h, pc.bytes, hipMemcpyHostToDevice, c->stream), "upload batch");
-        off += (pc.bytes + 255) / 256 * 256;
-    }
+    for (const Piece& pc : pieces)
+        if (pc.bytes) std::memcpy(static_cast<unsigned char*>(c->pinned) + pc.at, pc.src, pc.bytes);
+    hip_check(hipMemcpyAsync(w.in, c->pinned, total, hipMemcpyHostToDevice, c->stream), "upload batch");
     hip_check(hipEventRecord(c->staged_copy, c->stream), "hipEventRecord");
     c->staged_copy_recorded = true;
     set_staged(c, b, n, n_seqs, vectors);
@@ -1365,9 +1358,19 @@ void run_forward(ge_ctx* c, double* gpu_seconds, bool record_start) {
 }
 
 void read_pooled(ge_ctx* c, float* out) {
+    const size_t bytes = size_t(c->staged_seqs) * c->model.out_dims * 4;
+    if (bytes <= c->pinned_cap) {
+        // through the staging buffer, whose last upload is ahead of this copy on the stream: one wait
+        // for the forward and the copy together
+        hip_check(hipMemcpyAsync(c->pinned, c->ws.pooled, bytes, hipMemcpyDeviceToHost, c->stream), "read pooled");
+        hip_check(hipStreamSynchronize(c->stream), "hipStreamSynchronize");
+        std::memcpy(out, c->pinned, bytes);
+        if (c->prof) resolve_profile(c);
+        return;
+    }
     hip_check(hipStreamSynchronize(c->stream), "hipStreamSynchronize");
     if (c->prof) resolve_profile(c);
-    hip_check(hipMemcpy(out, c->ws.pooled, size_t(c->staged_seqs) * c->model.out_dims * 4, hipMemcpyDeviceToHost), "read pooled");
+    hip_check(hipMemcpy(out, c->ws.pooled, bytes, hipMemcpyDeviceToHost), "read pooled");
 }
 
 // Copies `rows` x `width` of a device buffer (fp32 or fp16, row stride `stride`) starting at

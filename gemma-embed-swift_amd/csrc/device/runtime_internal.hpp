@@ -76,14 +76,19 @@ struct Workspace {
     // qkv and t hold fp16 (scaled, see DevLayer::qkv_c) where the layer's kernels take it
     float *x = nullptr, *qkv = nullptr, *t = nullptr, *out = nullptr;
     uint16_t *h = nullptr, *q = nullptr, *k = nullptr, *v = nullptr, *attn = nullptr, *act = nullptr;
+    // The staged batch's small arrays (ids, positions, sequence ranges, work lists, V^T columns), one
+    // block uploaded by one copy; tokens ... work2 point into it, placed by stage() at 256-byte steps.
+    // Six copies of a few hundred bytes each took about 4 us of the GPU and 5 of the host apiece.
+    unsigned char* in = nullptr;
+    size_t in_cap = 0;
     int32_t *tokens = nullptr, *positions = nullptr;
-    int seq_cap = 0, work_cap = 0;
+    int seq_cap = 0;
     SeqRange* seqs = nullptr;
     AttnWork* work = nullptr;
     float* pooled = nullptr;
     // transposed V for the LDS-copy attention: vt [max_kvd][vt_cap], token t at column vcol[t];
     // its 64-query work list
-    int vt_cap = 0, work2_cap = 0;
+    int vt_cap = 0;
     uint16_t* vt = nullptr;
     int32_t* vcol = nullptr;
     AttnWork* work2 = nullptr;

@@ -139,18 +139,19 @@ def workspace(m, b):
     D = m["hidden"]
     ws = dict(x=R * D * F32, h=R * D * F16, qkv=R * m["max_qkv"] * F32, q=R * m["max_qd"] * F16,
               k=R * m["max_kvd"] * F16, v=R * m["max_kvd"] * F16, attn=R * m["max_qd"] * F16, t=R * D * F32,
-              act=R * m["ff"] * F16, out=R * m["out_dims"] * F32, hn=R * D * F32, tokens=R * I32, positions=R * I32,
-              vcol=R * I32)
+              act=R * m["ff"] * F16, out=R * m["out_dims"] * F32, hn=R * D * F32)
+    # one block uploaded by one copy (Workspace::in): each array at its exact size
+    ws.update(tokens=b["n"] * I32, positions=b["n"] * I32, vcol=b["n"] * I32)
     if m["any_precise"]:
         ws.update(h3=R * 3 * D * F16, q_lo=R * m["max_qd"] * F16, k_lo=R * m["max_kvd"] * F16)
     if m["pl"] > 0:
         ws.update(ple=R * m["layers"] * m["pl"] * F32, ple_t=R * max(m["pl"], D) * F32, rs=R * F32, rs2=R * F32,
                   x16=R * D * F16, g16=R * m["pl"] * F16)
     seq_cap = max(len(b["seqs"]), 1)
-    ws.update(seqs=seq_cap * SEQ_BYTES, pooled=seq_cap * m["out_dims"] * F32, pooled_n=seq_cap * D * F32,
-              work=max(len(b["work"]), 1) * WORK_BYTES)
+    ws.update(seqs=len(b["seqs"]) * SEQ_BYTES, pooled=seq_cap * m["out_dims"] * F32, pooled_n=seq_cap * D * F32,
+              work=0 if m["all_v2"] else len(b["work"]) * WORK_BYTES)
     if m["any_v2"]:
-        ws["work2"] = max(len(b["work2"]), 1) * WORK_BYTES
+        ws["work2"] = len(b["work2"]) * WORK_BYTES
         vt_cap = (b["vt_cols"] + 63) // 64 * 64
         ws["vt"] = m["max_kvd"] * vt_cap * F16
         b["vt_cap"] = vt_cap
@@ -362,7 +363,8 @@ def stage_copies(a, b):
     a.span("stage", ("tokens", 0), 0, n * I32)
     a.span("stage", ("positions", 0), 0, n * I32)
     a.span("stage", ("seqs", 0), 0, len(b["seqs"]) * SEQ_BYTES)
-    a.span("stage", ("work", 0), 0, len(b["work"]) * WORK_BYTES)
+    if a.sizes["work"]:  # staged only for layers off the LDS-copy attention
+        a.span("stage", ("work", 0), 0, len(b["work"]) * WORK_BYTES)
     if len(b["work2"]):
         a.span("stage", ("work2", 0), 0, len(b["work2"]) * WORK_BYTES)
         a.span("stage", ("vcol", 0), 0, n * I32)
