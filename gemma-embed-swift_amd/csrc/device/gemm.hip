@@ -837,14 +837,16 @@ hipError_t launch_gemm_q8(hipStream_t s, const Q8Dev& w, const uint16_t* x, int 
     // 24.4 -> 13.7; gate/up 2304 x 768 12.7 -> 8.3 at 1024 and 12.8 -> 9.2 at 1600. Past one round
     // of the 128 x 128 tiles the shapes below win again (gate/up at 2100 rows 13.0 against 13.9).
     // The two parts of a split forward choose by their own rows: counting both parts' tiles was
-    // slower (a 4096-token pack 2.27 against 2.09 ms, 8192 3.60 against 3.42).
+    // slower (a 4096-token pack 2.27 against 2.09 ms, 8192 3.60 against 3.42). Two parts of 2560 rows
+    // each take 480 tiles of 64 x 64 for o and down: 2.45 ms a pack, 2.59 with 240 of 64 x 128, whose
+    // 96 KB leave no room on a CU for the other part's.
     if (w.cols % 64 == 0) {
         const int64_t cus = g_wide_slots.load(std::memory_order_relaxed) / 2;
         const auto tiles = [&](int bm, int bn) { return int64_t((M + bm - 1) / bm) * ((w.rows + bn - 1) / bn); };
         if (epi != kEpiGeglu && w.cols % GemmMini::BK == 0 && tiles(64, 64) <= cus)
             return gemm_launch<GemmMini>(s, w, x, M, y, epi, out_scale, ea);
-        if (epi != kEpiGeglu && tiles(64, 64) <= cus * 7 / 4) return gemm_launch<GemmMini64>(s, w, x, M, y, epi, out_scale, ea);
-        if (tiles(64, 128) <= cus) return gemm_launch<GemmMid>(s, w, x, M, y, epi, out_scale, ea);
+        if (epi != kEpiGeglu && tiles(64, 64) <= cus * 2) return gemm_launch<GemmMini64>(s, w, x, M, y, epi, out_scale, ea);
+        if (epi == kEpiGeglu && tiles(64, 128) <= cus) return gemm_launch<GemmMid>(s, w, x, M, y, epi, out_scale, ea);
         if (tiles(128, 128) <= cus) return gemm_launch<GemmDeep>(s, w, x, M, y, epi, out_scale, ea);
     }
     // Tile shapes by projection and batch rows, from sweeps of the shapes (20 launches back to

@@ -8,9 +8,9 @@ import gemma_embed as ge
 pytestmark = pytest.mark.gpu
 
 # Rows at which a 768-wide projection changes shape on 256 CUs: the skinny kernel up to 320 (10 x 24
-# waves), 64 x 64 tiles up to 1344 (21 x 12) and, with fewer stages, up to 2368 (37 x 12), 64 x 128 up to
-# 2688 (42 x 6), 128 x 128 up to 5376 (42 x 6).
-EDGES = (1, 320, 321, 1344, 1345, 2368, 2369, 2688, 2689, 5376, 5377)
+# waves), 64 x 64 tiles up to 1344 (21 x 12) and, with shorter stages, up to 2688 (42 x 12), 128 x 128 up
+# to 5376 (42 x 6).
+EDGES = (1, 320, 321, 1344, 1345, 2688, 2689, 5376, 5377)
 # The same for gate/up pairs of 2304 columns: skinny up to 224 (7 x 36), 64 x 128 up to 896 (14 x 18),
 # 128 x 128 up to 1792 (14 x 18).
 PAIR_EDGES = (224, 225, 896, 897, 1792, 1793)
