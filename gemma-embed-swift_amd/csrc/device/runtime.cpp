@@ -1828,6 +1828,7 @@ void op_attention(ge_ctx* c, const void* q, const void* q_lo, const void* k, con
     std::vector<ge_attention_work> items(static_cast<size_t>(n_work), ge_attention_work{});
     hip_check(hipMemcpy(items.data(), work, items.size() * sizeof(ge_attention_work), hipMemcpyDeviceToHost), "read work");
     OpTemps temps(c);
+    std::vector<unsigned char> lists;  // outlives its upload (the synchronisation at the end)
     if (split || attention_v2_supported(head_dim, heads, kv_heads)) {
         // The sequences behind the work items, in order; V transposed into their layout.
         std::vector<ge_seq> seqs;
@@ -1848,15 +1849,19 @@ void op_attention(ge_ctx* c, const void* q, const void* q_lo, const void* k, con
             for (uint32_t q0 = 0; q0 < seqs[s].length; q0 += uint32_t(item_queries))
                 w2.push_back(AttnWork{seqs[s].start, seqs[s].length, q0, vl.start[s]});
         const int kvd = kv_heads * head_dim;
-        const size_t vt_at = temps.reserve(size_t(kvd) * vl.cols * 2), vcol_at = temps.reserve(size_t(T) * 4),
-                     dw_at = temps.reserve(w2.size() * sizeof(AttnWork));
+        // the V^T columns and the work list in one upload
+        const size_t col_bytes = (size_t(T) * 4 + 255) / 256 * 256, dw_bytes = w2.size() * sizeof(AttnWork);
+        lists.resize(col_bytes + dw_bytes);
+        std::memcpy(lists.data(), vl.vcol.data(), size_t(T) * 4);
+        if (dw_bytes) std::memcpy(lists.data() + col_bytes, w2.data(), dw_bytes);
+        const size_t vt_at = temps.reserve(size_t(kvd) * vl.cols * 2), lists_at = temps.reserve(lists.size());
         unsigned char* const base = temps.base();
         auto* vt = reinterpret_cast<uint16_t*>(base + vt_at);
-        auto* vcol = reinterpret_cast<int32_t*>(base + vcol_at);
-        auto* dw = reinterpret_cast<AttnWork*>(base + dw_at);
+        auto* vcol = reinterpret_cast<int32_t*>(base + lists_at);
+        auto* dw = reinterpret_cast<AttnWork*>(base + lists_at + col_bytes);
         hip_check(hipMemsetAsync(vt, 0, size_t(kvd) * vl.cols * 2, c->stream), "hipMemset");
-        hip_check(hipMemcpyAsync(vcol, vl.vcol.data(), size_t(T) * 4, hipMemcpyHostToDevice, c->stream), "upload");
-        hip_check(hipMemcpyAsync(dw, w2.data(), w2.size() * sizeof(AttnWork), hipMemcpyHostToDevice, c->stream), "upload");
+        if (!lists.empty())
+            hip_check(hipMemcpyAsync(vcol, lists.data(), lists.size(), hipMemcpyHostToDevice, c->stream), "upload");
         launch(c, "v_transpose", [&] {
             return launch_v_transpose(c->stream, static_cast<const uint16_t*>(v), T, kvd, vcol, vl.cols, vt);
         });
