@@ -630,8 +630,11 @@ hipError_t launch_mean_pool(hipStream_t s, const float* x, const SeqRange* seqs,
 // (dequantised once), then walks the workgroup's rows; each row's dot product is summed per lane
 // over its chunks in order, then over the lanes by a fixed butterfly, so a row's output depends
 // on that row alone.
-constexpr int kProjRows = 64;   // rows (sequences) per workgroup row of the grid
 constexpr int kProjUnroll = 8;  // rows whose loads are in flight together
+// Rows (sequences) per workgroup row of the grid: one batch of loads each, bound by their latency. With
+// 64 the batches ran one after another: 24 rows 10.2 -> 6.0 us, 32 13.4 -> 6.0, about 52 22.9 -> 8.3
+// (each workgroup dequantises its weights again, 0.6 MB a batch from L2).
+constexpr int kProjRows = kProjUnroll;
 
 template <int CH>
 __global__ __launch_bounds__(256) void pooled_projection_kernel(const float* __restrict__ in, int n_rows, int width,
