@@ -23,7 +23,7 @@ ATTN_QUERIES_V2 = 64     # kAttnQueriesV2, kernels.hpp:139
 SMALL_ITEMS = 256        # kAttnSmallItems, runtime.cpp
 SPLIT_MIN_TOKENS = 2048  # kSplitMinTokens, runtime_internal.hpp
 MAX_PARTS = 2            # kMaxParts, runtime_internal.hpp
-SKINNY_MAX_ROWS = 512    # kSkinnyMaxRows, kernels.hpp
+CUS = 256                # the skinny kernel takes launches of at most one wave per CU (skinny_ok, gemm.hip)
 WORK_BYTES, SEQ_BYTES = 16, 8  # sizeof(AttnWork), sizeof(SeqRange)
 
 
@@ -277,7 +277,7 @@ def gemm_qkv(a, M, N, K, hd, H, KV, x, e, pos, vc):
     if M == 0:
         return
     a.rsrc("gemm_qkv", x, 0, M * K * F16)
-    if e["stage"] is not None and M <= SKINNY_MAX_ROWS and K % 128 == 0:
+    if e["stage"] is not None and (M + 31) // 32 * (N // 32) <= CUS and K % 128 == 0:
         a.span("gemm_qkv (staging)", e["stage"], 0, M * N * F16)
     a.span("gemm_qkv", e["positions"], 0, M * I32)
     for p, heads in ((e["q"], H), (e["k"], KV), (e["v"], KV)):
