@@ -836,7 +836,8 @@ void stage(ge_ctx* c, const int32_t* tokens, const int32_t* positions, int n, co
                       // read only by layers off the LDS-copy attention
                       {b.work.data(), m.all_v2 ? 0 : b.work.size() * sizeof(AttnWork), 0},
                       {b.work2.data(), b.work2.size() * sizeof(AttnWork), 0},
-                      {b.vl.vcol.data(), b.work2.empty() ? 0 : size_t(n) * 4, 0}};
+                      // every token's, also where no sequence has any: the projections store each token's V
+                      {b.vl.vcol.data(), b.vl.vcol.size() * 4, 0}};
     size_t total = 0;
     for (Piece& pc : pieces) {
         pc.at = total;

@@ -1,0 +1,119 @@
+"""What the library enqueues and leaves behind, on the host HIP runtime (host_hip.cpp): run by
+tests/test_host_hip.py in a process of its own, whose GE_LIBRARY is the library's objects over it."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+import gemma_embed as ge
+
+P, I = C.c_void_p, C.c_int
+LAUNCH = C.CFUNCTYPE(None, C.c_char_p, C.POINTER(P))
+lib = ge.lib
+lib.host_hip_pending.restype = C.c_uint64
+lib.host_hip_pending_copies.restype = C.c_uint64
+lib.host_hip_pending_copies.argtypes = [P, C.c_size_t]
+lib.host_hip_block.argtypes = [P, C.POINTER(P), C.POINTER(C.c_size_t)]
+lib.host_hip_fail.argtypes = [C.c_char_p, I]
+lib.host_hip_on_launch.argtypes = [LAUNCH]
+
+
+class QkvEpilogue(C.Structure):
+    """kernels.hpp"""
+    _fields_ = [(n, P) for n in ("q_norm", "k_norm", "positions", "rope", "q", "k", "v", "vcol", "vt")] + \
+        [("scale", C.c_float), ("eps", C.c_float), ("vt_cols", I), ("heads", I), ("kv_heads", I), ("stage", P)]
+
+
+def arg(args, i, kind):
+    return C.cast(args[i], C.POINTER(kind))[0]
+
+
+def block_end(p):
+    """The end of the allocation p lies in."""
+    base, size = P(), C.c_size_t()
+    assert lib.host_hip_block(P(p), C.byref(base), C.byref(size)), hex(p)
+    return base.value + size.value
+
+
+def ints(p, n):
+    """n int32 of an array in device memory, which must hold them all."""
+    assert p + 4 * n <= block_end(p), f"{n} int32 at {p:#x} run past the allocation's end {block_end(p):#x}"
+    return np.ctypeslib.as_array(C.cast(p, C.POINTER(C.c_int32)), (n,)).copy()
+
+
+class Launches:
+    """The launches of a block, read as they are made: (kernel, what `read` returns) of those it knows.
+    A failing reader is raised when the block ends (ctypes callbacks swallow exceptions)."""
+
+    def __init__(self, read):
+        self.read, self.seen, self.error = read, [], None
+
+    def __enter__(self):
+        def on_launch(name, args):
+            try:
+                got = self.read(name.decode(), args)
+                if got is not None:
+                    self.seen.append((name.decode(), got))
+            except BaseException as e:  # noqa: BLE001
+                self.error = self.error or e
+        self.callback = LAUNCH(on_launch)
+        lib.host_hip_on_launch(self.callback)
+        return self.seen
+
+    def __exit__(self, *exc):
+        lib.host_hip_on_launch(LAUNCH())
+        if self.error and not exc[0]:
+            raise self.error
+
+
+def load(tmp_path, **shape):
+    path = ge.synth_write_gguf(str(tmp_path / "m.gguf"), **dict(ge.TINY, **shape))
+    return ge.EmbeddingModel.load(path)
+
+
+def vt_launch(name, args):
+    """(tokens, V^T columns of them, vt_cols) of a launch that stores V^T."""
+    if "gemm_qkv_kernel" in name or "qkv_rowpass_kernel" in name:
+        fused = "gemm_qkv_kernel" in name
+        n, e = arg(args, 2 if fused else 1, I), arg(args, 7 if fused else 3, QkvEpilogue)
+        vcol, cols, vt = e.vcol, e.vt_cols, e.vt
+        if not vt:
+            return None
+    elif "v_transpose_kernel" in name:
+        n, vcol, cols = arg(args, 1, I), arg(args, 3, P), arg(args, 4, I)
+    elif "qkv_norm_rope_vt_kernel" in name:
+        pytest.fail("a path these checks do not read")
+    else:
+        return None
+    return n, ints(vcol, n), cols
+
+
+# The QKV epilogue (from 65 rows in tiles, below as a row pass), and the separate V transpose of the
+# split-precision layers.
+SHAPES = {"fused": dict(heads=3, head_dim_swa=256, head_dim_global=256),
+          "transpose": dict(heads=4, head_dim_swa=512, head_dim_global=512)}
+
+
+@pytest.mark.parametrize("shape", SHAPES)
+def test_tokens_of_empty_sequences_have_v_columns(tmp_path, shape):
+    """A batch whose sequences are all empty still runs every token through the projections, which store
+    its V at vcol[token]: those columns must be there, inside V^T, whatever the batch before left."""
+    with load(tmp_path, **SHAPES[shape]) as model:
+        h = model.context.handle
+        ids = np.full(6000, 500, np.int32)
+        pos = (np.arange(6000) % 400).astype(np.int32)
+        out = np.zeros((8, model.context.out_dims), np.float32)
+
+        def forward(n, seqs):
+            with Launches(vt_launch) as seen:
+                model.context._check(lib.ge_forward(h, ge._ptr(ids, C.c_int32), ge._ptr(pos, C.c_int32), n,
+                                                    ge._seq_array(seqs), len(seqs), ge._ptr(out, C.c_float), None), "ge_forward")
+            assert sum(rows for _, (rows, _, _) in seen) == 2 * n  # two layers, every token
+            for name, (_, cols, vt_cols) in seen:
+                assert cols.min() >= 0 and cols.max() < vt_cols, (name, cols.min(), cols.max(), vt_cols)
+
+        forward(5000, [(0, 0)])            # a fresh workspace
+        forward(40, [(0, 0), (17, 0)])
+        forward(5999, [(0, 100), (200, 400)])  # the columns' place then holds other arrays' words
+        for n in (3, 64, 1000, 5000):
+            forward(n, [(0, 0), (1, 0)])

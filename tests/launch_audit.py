@@ -132,6 +132,14 @@ def plan(m, lengths, gaps=None):
     return b
 
 
+def staged_arrays(m, b):
+    """Bytes of each array stage() places in the block it uploads (Workspace::in). An access must stay inside
+    its own array, which is less than the block allows."""
+    return dict(tokens=b["n"] * I32, positions=b["n"] * I32, seqs=len(b["seqs"]) * SEQ_BYTES,
+                work=0 if m["all_v2"] else len(b["work"]) * WORK_BYTES, work2=len(b["work2"]) * WORK_BYTES,
+                vcol=0 if b["vcol"] is None else len(b["vcol"]) * I32)
+
+
 def workspace(m, b):
     """Allocation sizes of ensure_workspace_impl (runtime.cpp:617) for a staged batch (a fresh
     context: every capacity is the batch's own)."""
@@ -140,18 +148,15 @@ def workspace(m, b):
     ws = dict(x=R * D * F32, h=R * D * F16, qkv=R * m["max_qkv"] * F32, q=R * m["max_qd"] * F16,
               k=R * m["max_kvd"] * F16, v=R * m["max_kvd"] * F16, attn=R * m["max_qd"] * F16, t=R * D * F32,
               act=R * m["ff"] * F16, out=R * m["out_dims"] * F32, hn=R * D * F32)
-    # one block uploaded by one copy (Workspace::in): each array at its exact size
-    ws.update(tokens=b["n"] * I32, positions=b["n"] * I32, vcol=b["n"] * I32)
+    ws.update(staged_arrays(m, b))
     if m["any_precise"]:
         ws.update(h3=R * 3 * D * F16, q_lo=R * m["max_qd"] * F16, k_lo=R * m["max_kvd"] * F16)
     if m["pl"] > 0:
         ws.update(ple=R * m["layers"] * m["pl"] * F32, ple_t=R * max(m["pl"], D) * F32, rs=R * F32, rs2=R * F32,
                   x16=R * D * F16, g16=R * m["pl"] * F16)
     seq_cap = max(len(b["seqs"]), 1)
-    ws.update(seqs=len(b["seqs"]) * SEQ_BYTES, pooled=seq_cap * m["out_dims"] * F32, pooled_n=seq_cap * D * F32,
-              work=0 if m["all_v2"] else len(b["work"]) * WORK_BYTES)
+    ws.update(pooled=seq_cap * m["out_dims"] * F32, pooled_n=seq_cap * D * F32)
     if m["any_v2"]:
-        ws["work2"] = len(b["work2"]) * WORK_BYTES
         vt_cap = (b["vt_cols"] + 63) // 64 * 64
         ws["vt"] = m["max_kvd"] * vt_cap * F16
         b["vt_cap"] = vt_cap
@@ -357,27 +362,16 @@ def mean_pool(a, seqs, width, x, seq_ptr, pooled):
 
 # ---------------------------------------------------------------- the forward
 
-def stage_copies(a, b):
-    """The staged arrays stage() (runtime.cpp:837) copies into the workspace."""
-    n = b["n"]
-    a.span("stage", ("tokens", 0), 0, n * I32)
-    a.span("stage", ("positions", 0), 0, n * I32)
-    a.span("stage", ("seqs", 0), 0, len(b["seqs"]) * SEQ_BYTES)
-    if a.sizes["work"]:  # staged only for layers off the LDS-copy attention
-        a.span("stage", ("work", 0), 0, len(b["work"]) * WORK_BYTES)
-    if len(b["work2"]):
-        a.span("stage", ("work2", 0), 0, len(b["work2"]) * WORK_BYTES)
-        a.span("stage", ("vcol", 0), 0, n * I32)
-
-
 def replay(m, b, positions=None):
     """Replays the launches of one forward of batch b (encode, or encode_split when the plan splits
     it) and returns the Audit."""
     ws = workspace(m, b)
     a = Audit(ws)
-    stage_copies(a, b)
-    pos = positions if positions is not None else np.concatenate(
-        [np.arange(n) for _, n in b["seqs"]] + [np.zeros(0, np.int64)]).astype(np.int64)
+    pos = positions
+    if pos is None:
+        pos = np.zeros(b["n"], np.int64)
+        for s, n in b["seqs"]:
+            pos[s:s + n] = np.arange(n)
     if b["n_parts"] == 1:
         parts = [(0, b["n"], b["work2"], b["work"])]
     else:

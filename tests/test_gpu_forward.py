@@ -178,6 +178,31 @@ def test_split_batch_matches_single_stream(c2_model, config2_batch):
     assert np.array_equal(split, single)
 
 
+def test_tokens_of_empty_sequences(config2_gguf):
+    """Tokens that belong to no sequence run through the layers without attention work: empty sequences
+    pool to zeros, on a fresh workspace and after larger packs, whose vectors stay what they were."""
+    with ge.EmbeddingModel.load(config2_gguf) as m:
+        ctx = m.context
+        ids = ge.synth_tokens(61, 2, 262144, 5000)
+        pos = (np.arange(5000) % 1000).astype(np.int32)
+        pack = [ids[:700].tolist(), ids[700:1500].tolist()]
+
+        def empty(n):
+            print(f"{n} tokens, two empty sequences", flush=True)
+            out = np.full((2, 768), 7, np.float32)
+            ctx._check(ge.lib.ge_forward(ctx.handle, ge._ptr(ids, ge.C.c_int32), ge._ptr(pos, ge.C.c_int32), n,
+                                         ge._seq_array([(0, 0), (n // 2, 0)]), 2, ge._ptr(out, ge.C.c_float), None),
+                       "ge_forward")
+            assert not out.any()
+
+        empty(5000)
+        want, _ = ctx.forward(pack)
+        for n in (5000, 1500, 300, 40):
+            empty(n)
+            again, _ = ctx.forward(pack)
+            assert np.array_equal(again, want)
+
+
 @pytest.mark.timeout(300)
 def test_split_forward_repeats_bitwise(c2_model, config2_batch):
     """The pack split into parts on several streams, whose layers run unsynchronised on shared

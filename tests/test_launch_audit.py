@@ -1,8 +1,8 @@
 """CPU bounds audit of every kernel launch of the text forward (tests/launch_audit.py): for each
 synthetic model the GPU tests and the bench load and each pack shape they run, no access of any
 launch leaves its allocation. The planted-mistake cases check that the audit notices a workspace
-one row short, a V^T buffer one row short, slack-free legacy attention and the split forward's
-attention given plain row offsets instead of its part bases."""
+one row short, a V^T buffer one row short, V^T columns staged only beside attention work, slack-free
+legacy attention and the split forward's attention given plain row offsets instead of its part bases."""
 import numpy as np
 import pytest
 
@@ -53,6 +53,17 @@ def test_tokens_outside_every_sequence():
     assert not a.errors, "\n".join(a.errors[:10])
 
 
+@pytest.mark.parametrize("name", ["config2", "real_shapes"])
+def test_tokens_with_only_empty_sequences(name):
+    # no attention work at all, but every token's V is stored: its V^T column must have been staged
+    m = la.model_of(MODELS[name])
+    for n in (1, 300, 5000):
+        b = la.plan(m, [0, 0], gaps=[n, 0])
+        assert len(b["work2"]) == 0 and b["n"] == n
+        a = la.replay(m, b)
+        assert not a.errors, "\n".join(a.errors[:10])
+
+
 def test_split_plans_cover_all_work():
     for lengths in ([512] * 32, [1024] * 8, [7] * 600 + [4000], [3000, 5000, 192]):
         m = la.model_of(ge.CONFIG2)
@@ -97,6 +108,15 @@ def test_audit_reports_a_vt_buffer_one_row_short(monkeypatch):
     a = la.replay(m, b)
     assert any(e.startswith("attention: vt") for e in a.errors)
     assert any(e.startswith("gemm_qkv: vt") for e in a.errors)
+
+
+def test_audit_reports_columns_staged_only_with_work(monkeypatch):
+    real = la.staged_arrays
+    monkeypatch.setattr(la, "staged_arrays", lambda m, b: dict(real(m, b), **({} if len(b["work2"]) else {"vcol": 0})))
+    m = la.model_of(ge.CONFIG2)
+    assert not la.replay(m, la.plan(m, [40, 9])).errors
+    a = la.replay(m, la.plan(m, [0], gaps=[5000]))
+    assert any(e.startswith("gemm_qkv: vcol") for e in a.errors)
 
 
 def test_audit_reports_legacy_attention_without_row_slack(monkeypatch):
