@@ -44,6 +44,7 @@ struct VisionState {
     AttnWork* work = nullptr;
     // staged batch
     int staged_patches = -1, staged_tokens = 0, staged_work = 0;
+    bool patches_sent = true;  // whether every copy of the staged batch's patches has been enqueued
     int items = kAttnQueriesV2;  // query rows per attention work item of the staged batch
     // part p: patch rows [part_row[p], part_row[p + 1]) with work items [part_work[p], part_work[p + 1])
     int n_parts = 1, part_row[kMaxParts + 1] = {0}, part_work[kMaxParts + 1] = {0};
@@ -386,6 +387,7 @@ void vision_stage(ge_ctx* c, const float* patches, int n_patches, const ge_image
     for (const Piece& pc : pieces)
         if (pc.bytes) hip_check(hipMemcpy(pc.dst, pc.src, pc.bytes, hipMemcpyHostToDevice), "upload image batch");
     v.staged_patches = n_patches;
+    v.patches_sent = upload;
     v.staged_tokens = tokens;
     v.staged_work = int(work.size());
     v.items = items;
@@ -514,7 +516,8 @@ bool vision_layers(ge_ctx* c, const VitPart& p, VitStop* sp) {
 // overlap the other's work. host_patches: the batch's patches, still with the caller: each part's
 // are copied ahead of its own layers, the second part's while the first one runs; ev_start is
 // recorded after the first copy, so a call's GPU seconds start where the tower does. The caller
-// synchronises before it gives the memory back. Traced and profiled forwards run as one part.
+// synchronises before it gives the memory back, however this ends. Traced and profiled forwards run as
+// one part.
 void vision_encode(ge_ctx* c, VitStop* sp, const float* host_patches = nullptr) {
     VisionState& v = vision_of(c);
     if (v.staged_patches < 0) fail(GE_ERR_STATE, "no image batch is staged");
@@ -525,6 +528,7 @@ void vision_encode(ge_ctx* c, VitStop* sp, const float* host_patches = nullptr) 
         if (!host_patches) return;
         hip_check(hipMemcpyAsync(v.patches32 + size_t(r0) * v.area, host_patches + size_t(r0) * v.area,
                                  size_t(r1 - r0) * v.area * 4, hipMemcpyHostToDevice, to), "upload patches");
+        v.patches_sent = r1 == v.staged_patches;
         if (r0 == 0) hip_check(hipEventRecord(c->ev_start, to), "hipEventRecord");
     };
     if (v.n_parts == 1 || sp || c->prof) {
@@ -555,6 +559,14 @@ void vision_encode(ge_ctx* c, VitStop* sp, const float* host_patches = nullptr) 
     });
     if (stop("pooled", -1) || stop("pooled_normed", -1)) return;
     launch(c, "vit_gemm_proj", [&] { return launch_gemm_q8(s, v.proj_w, v.pooled16, T, v.out, kEpiF32); });
+}
+
+// Waits for the streams a tower's work may still be on, after a failure: the caller's memory must not be
+// read once the call has returned. A batch whose patches have not all been sent is dropped.
+void abandon_vision(ge_ctx* c) {
+    for (hipStream_t s : c->part_stream) (void)hipStreamSynchronize(s);
+    VisionState& v = vision_of(c);
+    if (!v.patches_sent) v.staged_patches = -1;
 }
 
 void vision_read(ge_ctx* c, float* out, size_t cap) {
@@ -741,15 +753,20 @@ int ge_vision_encode(ge_ctx* c, const float* patches, int32_t n_patches, const g
     if (!vectors) return GE_ERR_INVALID;
     return ge::guarded(c, [&] {
         ge::vision_stage(c, patches, n_patches, grids, n_images, false);
-        ge::vision_encode(c, nullptr, patches);
-        ge::hip_check(hipEventRecord(c->ev_stop, c->stream), "hipEventRecord");
-        if (gpu_seconds) {
-            ge::hip_check(hipEventSynchronize(c->ev_stop), "hipEventSynchronize");
-            float ms = 0;
-            ge::hip_check(hipEventElapsedTime(&ms, c->ev_start, c->ev_stop), "hipEventElapsedTime");
-            *gpu_seconds = ms * 1e-3;
+        try {
+            ge::vision_encode(c, nullptr, patches);
+            ge::hip_check(hipEventRecord(c->ev_stop, c->stream), "hipEventRecord");
+            if (gpu_seconds) {
+                ge::hip_check(hipEventSynchronize(c->ev_stop), "hipEventSynchronize");
+                float ms = 0;
+                ge::hip_check(hipEventElapsedTime(&ms, c->ev_start, c->ev_stop), "hipEventElapsedTime");
+                *gpu_seconds = ms * 1e-3;
+            }
+            ge::vision_read(c, vectors, vectors_count);
+        } catch (...) {
+            ge::abandon_vision(c);
+            throw;
         }
-        ge::vision_read(c, vectors, vectors_count);
     });
 }
 

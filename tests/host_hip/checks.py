@@ -117,3 +117,57 @@ def test_tokens_of_empty_sequences_have_v_columns(tmp_path, shape):
         forward(5999, [(0, 100), (200, 400)])  # the columns' place then holds other arrays' words
         for n in (3, 64, 1000, 5000):
             forward(n, [(0, 0), (1, 0)])
+
+
+@pytest.fixture(scope="module")
+def tower(tmp_path_factory):
+    path = ge.synth_write_vision_gguf(str(tmp_path_factory.mktemp("v") / "tower.gguf"), **ge.TINY_VISION)
+    ctx = ge.Context.create(0)
+    ctx.vision_load(path)
+    yield ctx
+    ctx.close()
+
+
+def vision_call(ctx, patches, grids, room):
+    """ge_vision_encode's status and message, with vectors of `room` floats."""
+    out = np.zeros(max(room, 1), np.float32)
+    rc = lib.ge_vision_encode(ctx.handle, ge._ptr(patches, C.c_float), len(patches), ge._grid_array(grids), len(grids),
+                              ge._ptr(out, C.c_float), room, None)
+    return rc, lib.ge_last_error(ctx.handle).decode()
+
+
+@pytest.mark.parametrize("images", [1, 30])  # one part; two (4320 patch rows)
+def test_failed_vision_encode_leaves_nothing_in_flight(tower, images):
+    """The images are copied from the caller's memory while the tower runs: whichever step fails, the call
+    waits for those copies, and a batch whose images did not all arrive is no longer staged."""
+    ctx, grids = tower, [(12, 12)] * images
+    patches = ge.image_patches(3, grids, ctx.vision_info().patch_area)
+    room = images * 16 * ctx.vision_info().proj_dims
+    assert vision_call(ctx, patches, grids, room)[0] == ge.GE_OK
+    nth_copy = images > 1 and 2 or 1
+    for call, n, arrived in ((b"hipMemcpyAsync", 1, False), (b"hipMemcpyAsync", nth_copy, False), (b"hipEventRecord", 2, None),
+                             (b"kernel:q8_fragments", 1, None), (b"kernel:gemm_kernel", 2 * images, None),
+                             (b"kernel:vit_residual2_ln", 5, None), (b"kernel:vit_pool", 1, True), (b"", 0, True)):
+        if call:
+            lib.host_hip_fail(call, n)
+        rc, message = vision_call(ctx, patches, grids, room if call else room - 1)
+        lib.host_hip_fail(call, 1 << 30)
+        if rc == ge.GE_OK:
+            assert arrived is None  # this batch does not make the call that often
+            continue
+        assert lib.host_hip_pending_copies(patches.ctypes.data, patches.nbytes) == 0, (call, message)
+        assert lib.host_hip_pending() == 0, (call, message)
+        if arrived is None:
+            arrived = lib.ge_vision_tokens(ctx.handle) >= 0
+        if arrived:  # a batch whose images are all there stays staged, and can be read or run again
+            if not call:
+                assert rc == ge.GE_ERR_INVALID and "vector buffer" in message
+                assert ctx.vision_read().size == room
+            ctx.vision_run()
+            ctx.sync()
+        else:
+            assert lib.ge_vision_tokens(ctx.handle) == -1
+            with pytest.raises(ge.GemmaEmbedError) as e:
+                ctx.vision_run()
+            assert e.value.code == ge.GE_ERR_STATE
+    assert vision_call(ctx, patches, grids, room)[0] == ge.GE_OK

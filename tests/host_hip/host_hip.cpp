@@ -40,7 +40,7 @@ std::map<const void*, void*>& vars() {  // host shadow -> block
     return m;
 }
 std::map<std::string, int> g_fail;  // call -> calls until it fails once
-hipError_t g_last = hipSuccess;
+hipError_t g_last = hipSuccess;      // set by failed launches only
 void (*g_on_launch)(const char*, void**) = nullptr;
 
 // Streams by id: operations issued, those known complete, and what each stream has waited for.
@@ -77,13 +77,9 @@ bool failing(const std::string& name) {
     g_fail.erase(it);
     return true;
 }
-hipError_t set(hipError_t e) {
-    if (e != hipSuccess) g_last = e;
-    return e;
-}
 hipError_t get_block(void** p, size_t n) {
     *p = std::calloc(n ? n : 1, 1);
-    if (!*p) return set(hipErrorOutOfMemory);
+    if (!*p) return hipErrorOutOfMemory;
     blocks()[reinterpret_cast<uintptr_t>(*p)] = n;
     return hipSuccess;
 }
@@ -96,7 +92,7 @@ hipError_t run_kernel(const void* f, void** args, hipStream_t s) {
     const std::string& name = kernels()[f];
     for (auto& kv : g_fail)
         if (kv.first.rfind("kernel:", 0) == 0 && name.find(kv.first.substr(7)) != std::string::npos) {
-            if (failing(std::string(kv.first))) return set(hipErrorLaunchFailure);
+            if (failing(std::string(kv.first))) return g_last = hipErrorLaunchFailure;
             break;
         }
     issue(s);
@@ -165,21 +161,21 @@ hipError_t hipGetLastError(void) {
     return e;
 }
 
-hipError_t hipMalloc(void** p, size_t n) { return failing("hipMalloc") ? set(hipErrorOutOfMemory) : get_block(p, n); }
+hipError_t hipMalloc(void** p, size_t n) { return failing("hipMalloc") ? hipErrorOutOfMemory : get_block(p, n); }
 hipError_t hipFree(void* p) { return p ? drop_block(p) : void(), hipSuccess; }
 hipError_t hipHostMalloc(void** p, size_t n, unsigned) {
-    return failing("hipHostMalloc") ? set(hipErrorOutOfMemory) : get_block(p, n);
+    return failing("hipHostMalloc") ? hipErrorOutOfMemory : get_block(p, n);
 }
 hipError_t hipHostFree(void* p) { return hipFree(p); }
-hipError_t hipGetSymbolAddress(void** p, const void* var) { return *p = vars()[var], *p ? hipSuccess : set(hipErrorInvalidSymbol); }
+hipError_t hipGetSymbolAddress(void** p, const void* var) { return *p = vars()[var], *p ? hipSuccess : hipErrorInvalidSymbol; }
 
 hipError_t hipMemcpy(void* d, const void* s, size_t n, hipMemcpyKind) {
-    if (failing("hipMemcpy")) return set(hipErrorInvalidValue);
+    if (failing("hipMemcpy")) return hipErrorInvalidValue;
     if (n) std::memcpy(d, s, n);
     return hipSuccess;
 }
 hipError_t hipMemcpyAsync(void* d, const void* s, size_t n, hipMemcpyKind kind, hipStream_t st) {
-    if (failing("hipMemcpyAsync")) return set(hipErrorInvalidValue);
+    if (failing("hipMemcpyAsync")) return hipErrorInvalidValue;
     if (n) std::memcpy(d, s, n);
     const uint64_t seq = issue(st);
     if (kind != hipMemcpyDeviceToDevice)
@@ -199,7 +195,7 @@ hipError_t hipStreamCreateWithFlags(hipStream_t* s, unsigned) {
 }
 hipError_t hipStreamDestroy(hipStream_t s) { return delete s, hipSuccess; }
 hipError_t hipStreamSynchronize(hipStream_t s) {
-    if (failing("hipStreamSynchronize")) return set(hipErrorUnknown);
+    if (failing("hipStreamSynchronize")) return hipErrorUnknown;
     merge(g_done, front(id_of(s)));
     return hipSuccess;
 }
@@ -208,17 +204,17 @@ hipError_t hipEventCreateWithFlags(hipEvent_t* e, unsigned) { return *e = new ih
 hipError_t hipEventCreate(hipEvent_t* e) { return *e = new ihipEvent_t, hipSuccess; }
 hipError_t hipEventDestroy(hipEvent_t e) { return delete e, hipSuccess; }
 hipError_t hipEventRecord(hipEvent_t e, hipStream_t s) {
-    if (failing("hipEventRecord")) return set(hipErrorUnknown);
+    if (failing("hipEventRecord")) return hipErrorUnknown;
     e->snap = front(id_of(s));
     return hipSuccess;
 }
 hipError_t hipEventSynchronize(hipEvent_t e) {
-    if (failing("hipEventSynchronize")) return set(hipErrorUnknown);
+    if (failing("hipEventSynchronize")) return hipErrorUnknown;
     return merge(g_done, e->snap), hipSuccess;
 }
 hipError_t hipEventQuery(hipEvent_t e) {
     for (size_t i = 0; i < e->snap.size(); i++)
-        if (e->snap[i] > slot(g_done, i)) return set(hipErrorNotReady);
+        if (e->snap[i] > slot(g_done, i)) return hipErrorNotReady;
     return hipSuccess;
 }
 hipError_t hipEventElapsedTime(float* ms, hipEvent_t, hipEvent_t) { return *ms = 1.0f, hipSuccess; }

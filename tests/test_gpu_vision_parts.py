@@ -34,3 +34,26 @@ def test_two_part_batches_bitwise(tiny_vision_gguf):
                 assert np.array_equal(alone, got[tok:tok + t]), i
             row, tok = row + n, tok + t
     ctx.close()
+
+
+@pytest.mark.parametrize("count", [1, 30])  # one part; two (4320 patch rows)
+def test_too_small_vector_buffer_leaves_the_patches_read(tiny_vision_gguf, count):
+    """A call that fails for its vector buffer has read the caller's patches when it returns: overwritten
+    after it, the batch still gives their vectors."""
+    ctx = ge.Context.create(0)
+    ctx.vision_load(tiny_vision_gguf)
+    patches, grids = batch([(12, 12)], count, 5)
+    want, _ = ctx.vision_encode(patches, grids)
+    for _ in range(3):
+        given = patches.copy()
+        out = np.zeros(want.size - 1, np.float32)
+        rc = ge.lib.ge_vision_encode(ctx.handle, ge._ptr(given, ge.C.c_float), len(given), ge._grid_array(grids), count,
+                                     ge._ptr(out, ge.C.c_float), out.size, None)
+        given[:] = 0.25
+        assert rc == ge.GE_ERR_INVALID
+        assert np.array_equal(ctx.vision_read(), want)
+        ctx.vision_run()
+        assert np.array_equal(ctx.vision_read(), want)
+        got, _ = ctx.vision_encode(patches, grids)
+        assert np.array_equal(got, want)
+    ctx.close()
