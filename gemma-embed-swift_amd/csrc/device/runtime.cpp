@@ -843,16 +843,13 @@ void stage(ge_ctx* c, const int32_t* tokens, const int32_t* positions, int n, co
         pc.at = total;
         total += (pc.bytes + 255) / 256 * 256;
     }
-    // The workspace may be reallocated below: nothing queued may still use it.
-    if (workspace_grows(c, n, n_seqs, total, b.vl.cols)) drain(c);
+    // The workspace may be reallocated below: nothing queued may still use it, and the batch staged before
+    // goes with its arrays. Until the new batch's upload a failure leaves that batch as it was otherwise.
+    if (workspace_grows(c, n, n_seqs, total, b.vl.cols)) {
+        drain(c);
+        c->staged_tokens = -1;
+    }
     ensure_workspace(c, n, n_seqs, total, b.vl.cols);
-    Workspace& w = c->ws;
-    w.tokens = reinterpret_cast<int32_t*>(w.in + pieces[0].at);
-    w.positions = reinterpret_cast<int32_t*>(w.in + pieces[1].at);
-    w.seqs = reinterpret_cast<SeqRange*>(w.in + pieces[2].at);
-    w.work = reinterpret_cast<AttnWork*>(w.in + pieces[3].at);
-    w.work2 = reinterpret_cast<AttnWork*>(w.in + pieces[4].at);
-    w.vcol = reinterpret_cast<int32_t*>(w.in + pieces[5].at);
     if (c->staged_copy_recorded) hip_check(hipEventSynchronize(c->staged_copy), "hipEventSynchronize");
     if (total > c->pinned_cap) {
         if (c->pinned) hip_check(hipHostFree(c->pinned), "hipHostFree");
@@ -864,6 +861,14 @@ void stage(ge_ctx* c, const int32_t* tokens, const int32_t* positions, int n, co
     }
     for (const Piece& pc : pieces)
         if (pc.bytes) std::memcpy(static_cast<unsigned char*>(c->pinned) + pc.at, pc.src, pc.bytes);
+    c->staged_tokens = -1;
+    Workspace& w = c->ws;
+    w.tokens = reinterpret_cast<int32_t*>(w.in + pieces[0].at);
+    w.positions = reinterpret_cast<int32_t*>(w.in + pieces[1].at);
+    w.seqs = reinterpret_cast<SeqRange*>(w.in + pieces[2].at);
+    w.work = reinterpret_cast<AttnWork*>(w.in + pieces[3].at);
+    w.work2 = reinterpret_cast<AttnWork*>(w.in + pieces[4].at);
+    w.vcol = reinterpret_cast<int32_t*>(w.in + pieces[5].at);
     hip_check(hipMemcpyAsync(w.in, c->pinned, total, hipMemcpyHostToDevice, c->stream), "upload batch");
     hip_check(hipEventRecord(c->staged_copy, c->stream), "hipEventRecord");
     c->staged_copy_recorded = true;

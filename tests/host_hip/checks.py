@@ -171,3 +171,39 @@ def test_failed_vision_encode_leaves_nothing_in_flight(tower, images):
                 ctx.vision_run()
             assert e.value.code == ge.GE_ERR_STATE
     assert vision_call(ctx, patches, grids, room)[0] == ge.GE_OK
+
+
+# (failing call, batch staged before, batch whose staging fails): in the workspace as it is, with the staged
+# block alone grown (as many tokens, more sequences), with everything grown and past the 1 MiB pinned buffer.
+STAGING_FAILURES = [(call, first, second) for call in (b"hipEventSynchronize", b"hipMemcpyAsync", b"hipEventRecord")
+                    for first, second in (([[5] * 700, [6] * 300], [[8] * 90]), ([[5] * 1000], [[6]] * 1000))] + \
+    [(b"hipHostMalloc", [[5] * 700, [6] * 300], [[7] * 1000] * 140), (b"hipMalloc", [[5] * 1000], [[6]] * 1000)]
+
+
+@pytest.mark.parametrize("call,first,second", STAGING_FAILURES)
+def test_failed_staging_keeps_no_mixed_batch(tmp_path, call, first, second):
+    """A staging that fails leaves either the batch before it, its arrays where its launches read them, or none."""
+    def read(name, args):
+        if "gemm_qkv_kernel" not in name and "qkv_rowpass_kernel" not in name:
+            return None
+        fused = "gemm_qkv_kernel" in name
+        n, e = arg(args, 2 if fused else 1, I), arg(args, 7 if fused else 3, QkvEpilogue)
+        return ints(e.positions, n).tolist() + ints(e.vcol, n).tolist()
+
+    with load(tmp_path, **SHAPES["fused"]) as model:
+        ctx = model.context
+        ctx.batch_stage(first)
+        with Launches(read) as before:
+            ctx.batch_run()
+        lib.host_hip_fail(call, 1)
+        with pytest.raises(ge.GemmaEmbedError) as e:
+            ctx.batch_stage(second)
+        assert e.value.code == ge.GE_ERR_GPU
+        with Launches(read) as after:
+            try:
+                ctx.batch_run()
+            except ge.GemmaEmbedError as failed:
+                assert failed.code == ge.GE_ERR_STATE
+        assert not after or after == before
+        ctx.batch_stage(second)
+        ctx.batch_run()
