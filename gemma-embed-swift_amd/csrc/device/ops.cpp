@@ -43,6 +43,9 @@ unsigned char* OpTemps::base() {
 }
 
 OpTemps::~OpTemps() {
+    // A call that fails after its first launch has not waited for it; the next call's constants are
+    // written by the host, in no order with the stream.
+    if (std::uncaught_exceptions() > unwinding_) (void)hipStreamSynchronize(c_->stream);
     if (c_->op_cap > kOpTempsKept) {
         (void)hipStreamSynchronize(c_->stream);
         (void)hipFree(c_->op_buf);

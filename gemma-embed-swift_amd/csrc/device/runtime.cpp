@@ -1833,8 +1833,8 @@ void op_attention(ge_ctx* c, const void* q, const void* q_lo, const void* k, con
     // The ABI's work items (ge_attention_work) come in; the kernels take ge::AttnWork.
     std::vector<ge_attention_work> items(static_cast<size_t>(n_work), ge_attention_work{});
     hip_check(hipMemcpy(items.data(), work, items.size() * sizeof(ge_attention_work), hipMemcpyDeviceToHost), "read work");
+    std::vector<unsigned char> lists;  // outlives its upload (the synchronisation at the end, or that of temps)
     OpTemps temps(c);
-    std::vector<unsigned char> lists;  // outlives its upload (the synchronisation at the end)
     if (split || attention_v2_supported(head_dim, heads, kv_heads)) {
         // The sequences behind the work items, in order; V transposed into their layout.
         std::vector<ge_seq> seqs;
@@ -1884,9 +1884,11 @@ void op_attention(ge_ctx* c, const void* q, const void* q_lo, const void* k, con
     } else {
         std::vector<AttnWork> w1;
         for (const auto& it : items) w1.push_back(AttnWork{it.seq_start, it.seq_len, it.q0, 0});
-        const size_t dw_at = temps.reserve(w1.size() * sizeof(AttnWork));
+        lists.resize(w1.size() * sizeof(AttnWork));
+        std::memcpy(lists.data(), w1.data(), lists.size());
+        const size_t dw_at = temps.reserve(lists.size());
         auto* dw = reinterpret_cast<AttnWork*>(temps.base() + dw_at);
-        hip_check(hipMemcpyAsync(dw, w1.data(), w1.size() * sizeof(AttnWork), hipMemcpyHostToDevice, c->stream), "upload");
+        hip_check(hipMemcpyAsync(dw, lists.data(), lists.size(), hipMemcpyHostToDevice, c->stream), "upload");
         launch(c, "attention", [&] {
             return launch_attention(c->stream, static_cast<const uint16_t*>(q), static_cast<const uint16_t*>(k),
                                     static_cast<const uint16_t*>(v), static_cast<uint16_t*>(out), dw, n_work, heads, kv_heads,

@@ -6,6 +6,7 @@
 
 #include <cstdint>
 #include <cstring>
+#include <exception>
 #include <map>
 #include <string>
 #include <utility>
@@ -237,7 +238,8 @@ int guarded(ge_ctx* c, F&& f) {
 void* dev_alloc(size_t bytes, const char* what);
 
 // Device memory for one per-op call's temporaries, the context's own from call to call: a call is
-// synchronous and a context's calls are serialised, so it is free again when the call returns.
+// synchronous, also when it fails, and a context's calls are serialised, so it is free again when the
+// call returns.
 // Allocating and freeing it per call took most of a small one: an attention call over 5132 rows
 // 142 us beside 42 us of kernels.
 constexpr size_t kOpTempsKept = size_t(64) << 20;
@@ -258,6 +260,7 @@ public:
 private:
     ge_ctx* c_;
     size_t used_ = 0;
+    const int unwinding_ = std::uncaught_exceptions();
 };
 hipEvent_t take_event(ge_ctx* c);
 

@@ -207,3 +207,23 @@ def test_failed_staging_keeps_no_mixed_batch(tmp_path, call, first, second):
         assert not after or after == before
         ctx.batch_stage(second)
         ctx.batch_run()
+
+
+@pytest.mark.parametrize("heads,head_dim", [(3, 256), (4, 256)])  # LDS-copy attention; the producer-wave one
+def test_refused_attention_call_leaves_nothing_in_flight(heads, head_dim):
+    """The per-op entries' temporaries are the context's: a call that is refused after its first kernel was
+    launched must have waited, or the next call's constants land in memory that kernel is still writing."""
+    ctx = ge.Context.create(0)
+    work = ge.attention_work([(0, 100), (100, 30)])
+    p = [ctx.alloc(n) for n in (200 * heads * head_dim * 2, 200 * head_dim * 2, 200 * head_dim * 2,
+                                200 * heads * head_dim * 2, work.nbytes)]
+    ctx.upload(p[4], work)
+    ctx.sync()
+    for half_window, scale_ok in ((-1, False), (0, True)):
+        try:
+            ctx.attention(p[0], p[1], p[2], p[3], p[4], len(work), heads, 1, head_dim, half_window)
+            assert scale_ok
+        except ge.GemmaEmbedError as e:
+            assert not scale_ok and e.code == ge.GE_ERR_INVALID
+        assert lib.host_hip_pending() == 0, half_window
+    ctx.close()

@@ -59,3 +59,28 @@ def test_calls_of_changing_sizes():
         print("embed", n, flush=True)
         embed(ctx, n, 1024, n)
     ctx.close()
+
+
+def test_norm_after_a_refused_attention_call():
+    """A call refused after its first launch has waited for it: the ones that the next norm takes for its
+    weights are not written over by that kernel."""
+    ctx = ge.Context.create(0)
+    attend(ctx, [4000], 1)  # sizes the temporaries
+    n, heads = 4000, 3
+    work = ge.attention_work([(0, n)])
+    big = [ctx.alloc((n + 64) * heads * 256 * 2) for _ in range(4)] + [ctx.alloc(work.nbytes)]
+    ctx.upload(big[2], np.full((n + 64, 256), 3.0, np.float16))
+    ctx.upload(big[4], work)
+    x = np.random.default_rng(2).standard_normal((64, 1024)).astype(np.float32)
+    px, out = ctx.alloc(x.nbytes), ctx.alloc(x.nbytes)
+    ctx.upload(px, x)
+    want = x / np.sqrt((x.astype(np.float64) ** 2).mean(axis=1, keepdims=True) + 1e-6)
+    for _ in range(5):
+        with pytest.raises(ge.GemmaEmbedError) as e:
+            ctx.attention(big[0], big[1], big[2], big[3], big[4], len(work), heads, 1, 256, -1)
+        assert e.value.code == ge.GE_ERR_INVALID
+        ctx.rmsnorm(px, out, None, 64, 1024, 1e-6)
+        assert np.abs(ctx.download(out, x.shape, np.float32) - want).max() < 1e-5
+    for p in big + [px, out]:
+        ctx.free(p)
+    ctx.close()
