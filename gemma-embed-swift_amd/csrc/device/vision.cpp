@@ -515,8 +515,9 @@ bool vision_layers(ge_ctx* c, const VitPart& p, VitStop* sp) {
 // runs as two parts on the context's two streams: one part's memory-bound passes and kernel tails
 // overlap the other's work. host_patches: the batch's patches, still with the caller: each part's
 // are copied ahead of its own layers, the second part's while the first one runs; ev_start is
-// recorded after the first copy, so a call's GPU seconds start where the tower does. The caller
-// synchronises before it gives the memory back, however this ends. Traced and profiled forwards run as
+// recorded after the first copy, so a call's GPU seconds start where the tower does and include what
+// the second part waits for its copy. The caller synchronises before it gives the memory back, however
+// this ends. Traced and profiled forwards run as
 // one part.
 void vision_encode(ge_ctx* c, VitStop* sp, const float* host_patches = nullptr) {
     VisionState& v = vision_of(c);

@@ -449,7 +449,8 @@ class Context:
     def vision_encode(self, patches: np.ndarray, grids: Sequence[Tuple[int, int]], proj_dims: Optional[int] = None,
                       merge: Optional[int] = None):
         """Patches [P, area] of images with the given grids -> (vectors [tokens, proj_dims], gpu_seconds).
-        The output is sized from the loaded tower; proj_dims and merge, when given, must match it."""
+        The output is sized from the loaded tower; proj_dims and merge, when given, must match it. From
+        4096 patches of several images, gpu_seconds includes what the second half's layers wait for its upload."""
         p, info = self._patches(patches)
         if (proj_dims is not None and proj_dims != info.proj_dims) or (merge is not None and merge != info.merge):
             raise GemmaEmbedError(GE_ERR_INVALID, f"the tower has merge {info.merge} and {info.proj_dims}-wide vectors")

@@ -288,7 +288,11 @@ int ge_vision_get_info(ge_ctx* ctx, ge_vision_info* info);
 
 /* VisionTower.upload + encode + read back: patches fp32 [n_patches][patch_area] -> vectors fp32
  * [tokens][proj_dims] (caller-owned, capacity vectors_count floats; tokens = sum of the images'
- * pooled tokens; GE_ERR_INVALID when it does not fit). Synchronous. */
+ * pooled tokens; GE_ERR_INVALID when it does not fit). Synchronous. `gpu_seconds` (nullable) receives
+ * the time from the tower's start on the GPU, once its first patches are there, to its last kernel. A
+ * batch of several images and at least 4096 patches uploads its second half while the first half's
+ * layers run: its time includes what those layers wait for that upload. ge_vision_run on a staged
+ * batch is the tower alone. */
 int ge_vision_encode(ge_ctx* ctx, const float* patches, int32_t n_patches, const ge_image_grid* grids, int32_t n_images,
                      float* vectors, size_t vectors_count, double* gpu_seconds);
 /* Device-resident image batches (as ge_batch_*): stage uploads the patches and descriptors, run
