@@ -788,6 +788,10 @@ BatchPlan plan_batch(ge_ctx* c, const int32_t* tokens, const int32_t* positions,
             b.n_parts = int(cuts.size()) + 1;
             for (int p = 1; p < b.n_parts; p++) b.part_row[p] = cuts[size_t(p) - 1];
             b.part_row[b.n_parts] = n;
+            for (int p = 0, parts = b.n_parts; p < parts; p++)
+                if (int64_t(b.part_row[p + 1] - b.part_row[p]) * kSplitMinShare < n) b.n_parts = 1;
+        }
+        if (b.n_parts > 1) {
             auto part_of = [&](const AttnWork& a) {
                 int p = 0;
                 while (p + 1 < b.n_parts && int(a.seq_start) >= b.part_row[p + 1]) p++;

@@ -347,10 +347,18 @@ struct StopPoint;
 void encode(ge_ctx* c, StopPoint* sp);
 // Waits for every stream of the context.
 void drain(ge_ctx* c);
-// Packs of at least this many tokens (of two or more sequences) run as parts on several streams:
-// 2048 tokens of 64 1.60 -> 1.45 ms, 3072 1.84 -> 1.69; at 1024 tokens one stream is faster (1.22
-// against 1.32 ms).
+// Packs of at least this many tokens (of two or more sequences) run as parts on several streams. One
+// stream / two parts, ms, config 2's model: 2048 tokens of 64 1.61 / 1.51, 4096 2.31 / 2.19, 8192
+// 3.51 / 3.13, 16384 5.62 / 5.29; at 1024 tokens one stream is faster (1.22 against 1.32). The reference's
+// architecture: 2048 2.36 / 2.46, 2500 of 200 3.09 / 2.93, 4096 3.50 / 3.30, 8192 5.36 / 5.42, 16384
+// 11.07 / 9.77. Its 2048 and 8192 lose 1-4% because the whole pack's launches fill their last round of
+// tiles there; the sizes between gain.
 constexpr int kSplitMinTokens = 2048;
+// A part has at least this fraction's share of the pack's tokens, else the pack runs on one stream. A
+// part of 5% lost 2-5% on both models at 2048 to 8000 tokens, of 12% -5% to 0, at [7, 2041] tokens 2.35 ms
+// on one stream and 2.42 on two (the reference's architecture 4.09 and 4.29); from 20% on it depends on how
+// both parts' launches round to tiles (-6% to +26% at 20%, -2% to +13% at 50%).
+constexpr int kSplitMinShare = 8;
 // The no-allocation forward takes packs below this many tokens.
 constexpr int kNoallocMaxTokens = 4096;
 // Takes the device address of the no-allocation forward's scratch array on the context's device

@@ -227,3 +227,15 @@ def test_refused_attention_call_leaves_nothing_in_flight(heads, head_dim):
             assert not scale_ok and e.code == ge.GE_ERR_INVALID
         assert lib.host_hip_pending() == 0, half_window
     ctx.close()
+
+
+@pytest.mark.parametrize("lengths,parts", [([1000, 1047], 1), ([1000, 1048], 2), ([7, 2041], 1), ([2041, 7], 1),
+                                           ([255, 1793], 1), ([256, 1792], 2), ([1792, 256], 2), ([1793, 255], 1),
+                                           ([3, 3000, 5], 1), ([600, 3000, 600], 2), ([64] * 40, 2)])
+def test_packs_split_only_into_parts_worth_a_stream(tmp_path, lengths, parts):
+    """From 2048 tokens, and only where the smaller part has an eighth of them."""
+    with load(tmp_path) as model:
+        with Launches(lambda name, args: arg(args, 3, I) if "embed_norm_kernel" in name else None) as seen:
+            model.context.forward([[5] * n for n in lengths])
+    rows = [n for _, n in seen]
+    assert len(rows) == parts and sum(rows) == sum(lengths) and min(rows) * 8 >= sum(lengths)

@@ -22,6 +22,7 @@ ATTN_QUERIES = 32        # kAttnQueries, kernels.hpp:26
 ATTN_QUERIES_V2 = 64     # kAttnQueriesV2, kernels.hpp:139
 SMALL_ITEMS = 256        # kAttnSmallItems, runtime.cpp
 SPLIT_MIN_TOKENS = 2048  # kSplitMinTokens, runtime_internal.hpp
+SPLIT_MIN_SHARE = 8      # kSplitMinShare, runtime_internal.hpp: a part has an eighth of the pack
 MAX_PARTS = 2            # kMaxParts, runtime_internal.hpp
 CUS = 256                # the skinny kernel takes launches of at most one wave per CU (skinny_ok, gemm.hip)
 WORK_BYTES, SEQ_BYTES = 16, 8  # sizeof(AttnWork), sizeof(SeqRange)
@@ -120,8 +121,8 @@ def plan(m, lengths, gaps=None):
                     best = x
             if 0 < best < n_tok:
                 cuts.append(best)
-        if cuts:
-            rows = [0] + cuts + [n_tok]
+        rows = [0] + cuts + [n_tok]
+        if cuts and min(np.diff(rows)) * SPLIT_MIN_SHARE >= n_tok:
             part = np.searchsorted(np.array(cuts), b["work2"][:, 0], side="right")
             order = np.argsort(part, kind="stable")
             counts = np.bincount(part, minlength=len(rows) - 1)

@@ -16,7 +16,7 @@ MODELS = {"tiny": ge.TINY, "tiny_ple": ge.TINY_PLE, "config2": ge.CONFIG2, "outl
 
 SHORT = [[1], [2], [40, 9], [63], [64], [65], [1] * 64, [5, 0, 7], [300], [1, 65], [100, 33, 7, 1]]
 LONG = [[1024] * 8, [512] * 32, [8192], [8192, 8192], [4096, 1], [1, 4096], [2048] * 8, [3000, 5000, 192],
-        [7] * 600 + [4000]]
+        [7] * 600 + [4000], [1000, 1047], [1000, 1048], [255, 1793], [256, 1792], [1800, 257], [7, 2500], [64] * 41]
 
 
 def config3_batches():
@@ -65,7 +65,7 @@ def test_tokens_with_only_empty_sequences(name):
 
 
 def test_split_plans_cover_all_work():
-    for lengths in ([512] * 32, [1024] * 8, [7] * 600 + [4000], [3000, 5000, 192]):
+    for lengths in ([512] * 32, [1024] * 8, [7] * 600 + [4000], [3000, 5000, 192], [256, 1792], [1000, 1048], [64] * 41):
         m = la.model_of(ge.CONFIG2)
         b = la.plan(m, lengths)
         assert b["n_parts"] > 1
@@ -73,6 +73,12 @@ def test_split_plans_cover_all_work():
         for p in range(b["n_parts"]):
             w = b["work2"][b["part_work"][p]:b["part_work"][p + 1]]
             assert np.all(w[:, 0] >= b["part_row"][p]) and np.all(w[:, 0] + w[:, 1] <= b["part_row"][p + 1])
+
+
+def test_packs_with_a_short_part_are_not_split():
+    m = la.model_of(ge.CONFIG2)
+    for lengths in ([1000, 1047], [7, 2500], [255, 1793], [1793, 255], [4096, 1], [1, 4096]):
+        assert la.plan(m, lengths)["n_parts"] == 1, lengths
 
 
 # ---- planted mistakes: each must be reported
