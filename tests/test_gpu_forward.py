@@ -155,9 +155,9 @@ def test_every_trace_tensor_vs_oracle(c2_model, c2_oracle, config2_batch, length
 
 
 def test_split_batch_matches_single_stream(c2_model, config2_batch):
-    """A pack of >= 4096 tokens runs as two halves of whole sequences on two streams; with
-    profiling on, the same pack runs on one stream. Same kernels on the same rows: the vectors
-    must be identical."""
+    """A pack of >= 2048 tokens runs as two parts of whole sequences on two streams; with
+    profiling on, the same pack runs on one stream. The tile shapes follow each launch's rows, the
+    arithmetic of a row does not: the vectors must be identical."""
     ctx = c2_model.context
     print("config2 pack of 16384: two streams vs one", flush=True)
     split, _ = ctx.forward(config2_batch)
@@ -176,6 +176,29 @@ def test_split_batch_matches_single_stream(c2_model, config2_batch):
     finally:
         ctx.profile_disable()
     assert np.array_equal(split, single)
+
+
+# the split's first sizes, evenly cut and as unevenly as it cuts (a part of an eighth: its o and down
+# projections on the skinny kernel, the other's on tiles), and packs just short of either
+SPLIT_EDGES = [[1000, 1047], [1000, 1048], [255, 1793], [256, 1792], [1792, 256], [330, 2301], [2300, 341], [7, 2500],
+               [64] * 47, [200] * 13]
+
+
+@pytest.mark.timeout(300)
+@pytest.mark.parametrize("which", ["config2", "real_shapes"])
+def test_first_split_sizes_match_single_stream(which, config2_gguf, real_shapes_gguf):
+    with ge.EmbeddingModel.load(config2_gguf if which == "config2" else real_shapes_gguf) as m:
+        ctx = m.context
+        for lengths in SPLIT_EDGES:
+            print(f"{which}: {len(lengths)} texts, {sum(lengths)} tokens", flush=True)
+            seqs = [ge.synth_tokens(70 + i, 2, 262144, n).tolist() for i, n in enumerate(lengths)]
+            split, _ = ctx.forward(seqs)
+            ctx.profile_enable("")
+            try:
+                single, _ = ctx.forward(seqs)
+            finally:
+                ctx.profile_disable()
+            assert np.array_equal(split, single), lengths
 
 
 def test_tokens_of_empty_sequences(config2_gguf):
@@ -723,7 +746,7 @@ def test_reference_real_architecture_vs_oracle(real_shapes_gguf):
 
 @pytest.mark.timeout(300)
 def test_reference_real_architecture_split_pack_bitwise(real_shapes_gguf):
-    """A pack of at least 4096 tokens runs as parts on several streams, through every layer type
+    """A pack of at least 2048 tokens runs as parts on two streams, through every layer type
     of the real architecture (fused and fp32 QKV, head dims 256 and 512, the per-layer-input
     branch): each text must have the bits it has alone (one stream)."""
     m = ge.EmbeddingModel.load(real_shapes_gguf, batch_token_budget=16384)

@@ -41,6 +41,20 @@ def test_no_alloc_forward_matches_forward(which, config2_gguf, real_shapes_gguf)
         m.close()
 
 
+def test_no_alloc_forward_of_packs_the_forward_splits(config2_gguf):
+    """From 2048 tokens of several texts ge_forward runs two parts; the no-allocation forward keeps one
+    stream, over the same plan."""
+    with ge.EmbeddingModel.load(config2_gguf) as m:
+        ctx = m.context
+        for lengths in ([1000, 1047], [1000, 1048], [1792, 256], [256, 1792], [7, 2500], [300, 2301], [64] * 40):
+            print(f"{len(lengths)} texts, {sum(lengths)} tokens", flush=True)
+            seqs = [ge.synth_tokens(120 + i, 2, 262144, n).tolist() for i, n in enumerate(lengths)]
+            want, _ = ctx.forward(seqs)
+            for _ in range(2):
+                got, _ = ctx.forward_noalloc(seqs)
+                assert np.array_equal(got, want), lengths
+
+
 def test_no_alloc_forward_refuses_what_does_not_fit(config2_gguf):
     m = ge.EmbeddingModel.load(config2_gguf)
     try:
