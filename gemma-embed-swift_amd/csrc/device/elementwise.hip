@@ -627,14 +627,13 @@ hipError_t launch_mean_pool(hipStream_t s, const float* x, const SeqRange* seqs,
 // per token, and in fp32 throughout: the Q8_0 weights as d * q (exact in fp32) and the normed rows
 // as the final norm computed them, where the token-wise GEMM rounds both to fp16.
 // One wave per output column n: lane l holds columns c * 256 + 4 l .. + 3 of the weight row
-// (dequantised once), then walks the workgroup's rows; each row's dot product is summed per lane
+// (dequantised once) for the workgroup's kProjRows rows; each row's dot product is summed per lane
 // over its chunks in order, then over the lanes by a fixed butterfly, so a row's output depends
 // on that row alone.
-constexpr int kProjUnroll = 8;  // rows whose loads are in flight together
-// Rows (sequences) per workgroup row of the grid: one batch of loads each, bound by their latency. With
-// 64 the batches ran one after another: 24 rows 10.2 -> 6.0 us, 32 13.4 -> 6.0, about 52 22.9 -> 8.3
+// Rows (sequences) per workgroup row of the grid: one batch of loads, bound by their latency. With 64,
+// eight such batches ran one after another: 24 rows 10.2 -> 6.0 us, 32 13.4 -> 6.0, about 52 22.9 -> 8.3
 // (each workgroup dequantises its weights again, 0.6 MB a batch from L2).
-constexpr int kProjRows = kProjUnroll;
+constexpr int kProjRows = 8;
 
 template <int CH>
 __global__ __launch_bounds__(256) void pooled_projection_kernel(const float* __restrict__ in, int n_rows, int width,
@@ -643,7 +642,7 @@ __global__ __launch_bounds__(256) void pooled_projection_kernel(const float* __r
                                                                 float* __restrict__ out) {
     const int n = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
     if (n >= n_out) return;
-    const int r0 = blockIdx.y * kProjRows, r1 = min(r0 + kProjRows, n_rows);
+    const int r0 = blockIdx.y * kProjRows;
     float wv[CH][4];
 #pragma unroll
     for (int c = 0; c < CH; c++) {
@@ -652,30 +651,28 @@ __global__ __launch_bounds__(256) void pooled_projection_kernel(const float* __r
         const float dsc = h2f(sc[(size_t)n * (width / 32) + ec / 32]);
         wv[c][0] = dsc * float(q4.x), wv[c][1] = dsc * float(q4.y), wv[c][2] = dsc * float(q4.z), wv[c][3] = dsc * float(q4.w);
     }
-    // kProjUnroll rows at a time, all their loads issued before any product (rows past r1 re-read
-    // row r1 - 1, unused), so the loop waits for one batch of loads rather than for each row's
-    for (int r = r0; r < r1; r += kProjUnroll) {
-        float4 xa[kProjUnroll][CH];
+    // all the rows' loads issued before any product (rows past the last re-read it, unused), so the
+    // workgroup waits for one batch of loads rather than for each row's
+    float4 xa[kProjRows][CH];
 #pragma unroll
-        for (int u = 0; u < kProjUnroll; u++)
+    for (int u = 0; u < kProjRows; u++)
 #pragma unroll
-            for (int c = 0; c < CH; c++)
-                xa[u][c] = *reinterpret_cast<const float4*>(in + (size_t)min(r + u, r1 - 1) * width +
-                                                            min(c * 256 + lane * 4, width - 4));
+        for (int c = 0; c < CH; c++)
+            xa[u][c] = *reinterpret_cast<const float4*>(in + (size_t)min(r0 + u, n_rows - 1) * width +
+                                                        min(c * 256 + lane * 4, width - 4));
 #pragma unroll
-        for (int u = 0; u < kProjUnroll; u++) {
-            float acc = 0.0f;
+    for (int u = 0; u < kProjRows; u++) {
+        float acc = 0.0f;
 #pragma unroll
-            for (int c = 0; c < CH; c++)
-                if (c * 256 + lane * 4 < width) {
-                    acc = __builtin_fmaf(xa[u][c].x, wv[c][0], acc);
-                    acc = __builtin_fmaf(xa[u][c].y, wv[c][1], acc);
-                    acc = __builtin_fmaf(xa[u][c].z, wv[c][2], acc);
-                    acc = __builtin_fmaf(xa[u][c].w, wv[c][3], acc);
-                }
-            acc = wave_sum(acc);
-            if (lane == 0 && r + u < r1) out[(size_t)(r + u) * n_out + n] = acc;
-        }
+        for (int c = 0; c < CH; c++)
+            if (c * 256 + lane * 4 < width) {
+                acc = __builtin_fmaf(xa[u][c].x, wv[c][0], acc);
+                acc = __builtin_fmaf(xa[u][c].y, wv[c][1], acc);
+                acc = __builtin_fmaf(xa[u][c].z, wv[c][2], acc);
+                acc = __builtin_fmaf(xa[u][c].w, wv[c][3], acc);
+            }
+        acc = wave_sum(acc);
+        if (lane == 0 && r0 + u < n_rows) out[(size_t)(r0 + u) * n_out + n] = acc;
     }
 }
 

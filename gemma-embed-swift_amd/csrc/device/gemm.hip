@@ -141,7 +141,7 @@ using GemmSquare = GemmCfg<256, 256, 4, 4, 64, 2>;
 using GemmSmall = GemmCfg<128, 128, 2, 2, 64, 2>;
 // Launches whose tiles of the shapes above would leave most of the CUs idle take smaller tiles and
 // deeper stage rings (one or two workgroups a CU, so the ring, not the neighbours, covers the
-// copies' latency); gemm_shape holds the rule and what it measured.
+// copies' latency); launch_gemm_q8 holds the rule and what it measured.
 using GemmMini = GemmCfg<64, 64, 2, 2, 128, 3>;
 using GemmMini64 = GemmCfg<64, 64, 2, 2, 64, 3>;
 using GemmMid = GemmCfg<64, 128, 2, 2, 64, 4>;
