@@ -135,9 +135,8 @@ def test_every_trace_tensor_vs_oracle(c2_model, c2_oracle, config2_batch, length
     """Every named intermediate the C-ABI traces (llama.cpp names), at a sliding (0) and a global (5)
     layer, against the oracle on the middle text of a pack: the embedding, the norms, the raw and
     the normed/rotated projections, attention, the GeGLU product, the FFN output, the layer output
-    and the final norm and projection. A pack of at most 512 tokens runs its GEMMs on the skinny
-    kernel (the mid pack: 201 rows, a partial last row block), one of at most 64 also replays as a
-    graph (short)."""
+    and the final norm and projection. The mid pack's 201 rows (a partial last row block) run on the
+    skinny kernel but for the 1280-wide QKV (280 of its blocks for 256 CUs), the short pack's all do."""
     batch = [config2_batch[2 + 4 * i][:n] for i, n in enumerate(lengths)]
     idx, lo = 1, lengths[0]
     per_layer = ["attn_norm", "Qcur", "Kcur", "Vcur", "Qcur_pos", "Kcur_pos", "Vcur_normed", "kqv_out",
@@ -342,14 +341,15 @@ def test_packing_invariance_and_determinism(c2_model, config2_batch):
 
 
 def test_short_texts_alone_match_larger_packs(c2_model, config2_batch):
-    """A pack of at most 512 tokens runs its GEMMs on the skinny kernel and the QKV epilogue as a
-    separate row pass (and, up to 64 tokens, replays as a graph); inside a pack of more than 512
-    tokens the same text runs on the tiled kernels. The vector must have the same bits either
-    way (MetalForwardTests.swift:95-120: counts around the tile boundaries, alone and between a
-    19- and a 500-token text)."""
+    """Alone, a text of up to 192 tokens runs all its GEMMs on the skinny kernel and the QKV epilogue as a
+    separate row pass (and, up to 64 tokens, replays as a graph), one of up to 320 its o and down
+    projections; inside a pack of more than 512 tokens the same text runs on the tiled kernels. The vector
+    must have the same bits either way (MetalForwardTests.swift:95-120: counts around the tile boundaries,
+    alone and between a 19- and a 500-token text)."""
     body = config2_batch[7]
     ctx = c2_model.context
-    for count in (1, 2, 13, 15, 16, 17, 31, 32, 33, 63, 64, 65, 127, 128, 129, 255, 256, 257, 480, 511, 512):
+    for count in (1, 2, 13, 15, 16, 17, 31, 32, 33, 63, 64, 65, 127, 128, 129, 192, 193, 255, 256, 257, 320, 321, 480, 511,
+                  512):
         subject = body[:count]
         packed, _ = ctx.forward([config2_batch[3][:19], subject, config2_batch[4][:500]])
         alone, _ = ctx.forward([subject])

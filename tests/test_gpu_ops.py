@@ -103,14 +103,16 @@ def test_gemm_f16_output_and_row_independence(ctx, c2):
 def test_gemm_row_boundaries_bitwise(ctx, c2, name):
     """The reference's batch-register GEMM check (BatchRegisterGemmTests.swift:81-137): a row's
     result is the same bits at every batch size. The 768-wide projections change kernel and tile
-    with the row count (skinny up to 512, 128 x 128 below 6144, 128 x 256 below 12288, 256 x 192
-    from there); each batch below is compared with the same rows of a 16384-row launch."""
+    with the row count on 256 CUs (skinny up to 320, 64 x 64 in deep stages up to 1344 and in shorter
+    ones up to 2688, 128 x 128 in three stages up to 5376 and in two below 6144, 128 x 256 below 12288,
+    256 x 192 from there); each batch below is compared with the same rows of a 16384-row launch."""
     shape, _, _ = c2.tensors[name]
     cols, rows = shape
     raw = np.asarray(c2.raw(name))
     x16 = f16_round(RNG.standard_normal((16384, cols)))
     full = run_gemm(ctx, raw, rows, cols, x16, y_f16=True)
-    for M in (1, 63, 64, 65, 511, 512, 513, 2047, 2048, 2049, 6143, 6144, 8192, 12287, 12288, 12289):
+    for M in (1, 63, 64, 65, 320, 321, 511, 512, 513, 1344, 1345, 2047, 2048, 2049, 2688, 2689, 5376, 5377, 6143, 6144,
+              8192, 12287, 12288, 12289):
         lo = min(777, 16384 - M)
         print(f"{name}: rows [{lo}, {lo + M}) against the 16384-row launch", flush=True)
         part = run_gemm(ctx, raw, rows, cols, x16[lo:lo + M].copy(), y_f16=True)
@@ -120,14 +122,14 @@ def test_gemm_row_boundaries_bitwise(ctx, c2, name):
 @pytest.mark.parametrize("name,y_f16", [("blk.1.attn_q.weight", False), ("blk.1.ffn_down.weight", True),
                                          ("output.weight", False)])
 def test_gemm_short_batches_match_tiled_rows(ctx, c2, name, y_f16):
-    """Up to 512 rows run on the skinny kernel; the same rows inside a 600-row batch run on the
-    tiled kernel. Same MFMA, operand order and k order: the same bits."""
+    """Up to 320 rows (of 768 columns: one 32 x 32 block per CU) run on the skinny kernel; the same rows
+    inside a 600-row batch run on the tiled kernel. Same MFMA, operand order and k order: the same bits."""
     shape, _, _ = c2.tensors[name]
     cols, rows = shape
     raw = np.asarray(c2.raw(name))
     x16 = f16_round(RNG.standard_normal((600, cols)))
     full = run_gemm(ctx, raw, rows, cols, x16, y_f16)
-    for lo, n in ((0, 1), (5, 7), (100, 32), (200, 33), (236, 64), (88, 300), (50, 512)):
+    for lo, n in ((0, 1), (5, 7), (100, 32), (200, 33), (236, 64), (88, 300), (40, 320), (40, 321), (50, 512)):
         part = run_gemm(ctx, raw, rows, cols, x16[lo:lo + n].copy(), y_f16)
         assert np.array_equal(full[lo:lo + n], part), (lo, n)
 
