@@ -2,9 +2,9 @@
 
 For every kernel the forward launches, this module restates the index arithmetic by which the
 kernel's threads address global memory, the workspace the runtime allocates for a batch
-(ensure_workspace_impl, csrc/device/runtime.cpp:617), the batch plan it stages (plan_batch :724,
-vt_layout :703, stage :837) and the launch sequence with its pointer arguments (encode :915 for one
-stream, encode_split :1051 for a batch split over streams, both ending in encode_tail :904). Every access range of every launch is
+(ensure_workspace_impl, csrc/device/runtime.cpp), the batch plan it stages (plan_batch,
+vt_layout, stage) and the launch sequence with its pointer arguments (encode for one
+stream, encode_split for a batch split over streams, both ending in encode_tail). Every access range of every launch is
 checked against the allocation its pointer falls in.
 
 - Plain loads and stores: the range of element indices the kernel's guards let through.
@@ -17,9 +17,9 @@ Sizes are in bytes; a pointer is (buffer name, byte offset)."""
 import numpy as np
 
 F32, F16, I32 = 4, 2, 4
-ROW_SLACK = 256          # kRowSlack, csrc/device/kernels.hpp:29
-ATTN_QUERIES = 32        # kAttnQueries, kernels.hpp:26
-ATTN_QUERIES_V2 = 64     # kAttnQueriesV2, kernels.hpp:139
+ROW_SLACK = 256          # kRowSlack, csrc/device/kernels.hpp
+ATTN_QUERIES = 32        # kAttnQueries, kernels.hpp
+ATTN_QUERIES_V2 = 64     # kAttnQueriesV2, kernels.hpp
 SMALL_ITEMS = 256        # kAttnSmallItems, runtime.cpp
 SPLIT_MIN_TOKENS = 2048  # kSplitMinTokens, runtime_internal.hpp
 SPLIT_MIN_SHARE = 8      # kSplitMinShare, runtime_internal.hpp: a part has an eighth of the pack
@@ -31,7 +31,7 @@ WORK_BYTES, SEQ_BYTES = 16, 8  # sizeof(AttnWork), sizeof(SeqRange)
 # ---------------------------------------------------------------- model
 
 def v2_supported(hd, H, KV):
-    """attention_v2_supported (csrc/device/attention.hip:808)."""
+    """attention_v2_supported (csrc/device/attention.hip)."""
     if hd == 512:
         return KV > 0 and H == 4 * KV
     if not (hd in (128, 256) and KV > 0 and H % KV == 0 and 1 <= H // KV <= 4):
@@ -41,7 +41,7 @@ def v2_supported(hd, H, KV):
 
 
 def model_of(spec):
-    """The device model's shape and per-layer path flags, as upload() (runtime.cpp:450) derives them
+    """The device model's shape and per-layer path flags, as upload() (runtime.cpp) derives them
     from a synthetic model spec (gemma_embed.synth_write_gguf's keyword arguments)."""
     H, D = spec["heads"], spec["hidden"]
     m = dict(layers=spec["layers"], hidden=D, heads=H, ff=spec["feed_forward"], out_dims=spec["out_dims"],
@@ -56,7 +56,7 @@ def model_of(spec):
         sl = H + 2 * KV
         L = dict(sliding=sliding, hd=hd, kv=KV, qd=H * hd, kvd=KV * hd)
         # hd >= ge_ctx::split_head_dim (512, or 0 after ge_set_split_scores(ctx, 0)) and
-        # attention_split_supported (attention.hip:1073)
+        # attention_split_supported (attention.hip)
         split_ok = (hd == 512 and H == 4 * KV) or (hd == 256 and H == 3 * KV)
         L["precise"] = split_ok and hd >= (0 if spec.get("split_scores") else 512)
         L["attn_v2"] = v2_supported(hd, H, KV)
@@ -80,9 +80,9 @@ def model_of(spec):
 # ---------------------------------------------------------------- batch plan and workspace
 
 def plan(m, lengths, gaps=None):
-    """plan_batch (runtime.cpp:724) for sequences of the given lengths packed back to back (with
+    """plan_batch (runtime.cpp) for sequences of the given lengths packed back to back (with
     `gaps[i]` unused rows before sequence i): sequence ranges, both attention work lists as arrays
-    of (seq_start, seq_len, q0, vt_start), the V^T layout (vt_layout :703) and the split into parts."""
+    of (seq_start, seq_len, q0, vt_start), the V^T layout (vt_layout) and the split into parts."""
     starts, r = [], 0
     for i, n in enumerate(lengths):
         r += gaps[i] if gaps else 0
@@ -142,7 +142,7 @@ def staged_arrays(m, b):
 
 
 def workspace(m, b):
-    """Allocation sizes of ensure_workspace_impl (runtime.cpp:617) for a staged batch (a fresh
+    """Allocation sizes of ensure_workspace_impl (runtime.cpp) for a staged batch (a fresh
     context: every capacity is the batch's own)."""
     R = (b["n"] + 63) // 64 * 64 + ROW_SLACK
     D = m["hidden"]
@@ -200,8 +200,8 @@ def at(ptr, nbytes):
 # ---------------------------------------------------------------- kernels
 
 def row_kernel(a, kernel, T, spans):
-    """The one-wave-per-row kernels (embed_norm_kernel elementwise.hip:15, residual_norm_kernel :120,
-    norm_split_kernel :264, the ple_*_kernel family ple.hip:30-218): row < T; loads of chunk
+    """The one-wave-per-row kernels (embed_norm_kernel elementwise.hip, residual_norm_kernel,
+    norm_split_kernel, the ple_*_kernel family ple.hip): row < T; loads of chunk
     min(e, width - 4) and stores of element e = c * 256 + 4 lane + j < width. spans: (pointer, bytes
     per row of the access)."""
     for ptr, row_bytes in spans:
@@ -222,7 +222,7 @@ def norm_split(a, T, D, x, h3):
 
 
 def qk_norm_rope(a, T, H, KV, HD, qkv, positions, q, k, v, q_lo=None, k_lo=None, pos=None, table_rows=8192):
-    """qk_norm_rope_kernel (elementwise.hip:327): item = (t, slot) < T (H + 2 KV); reads
+    """qk_norm_rope_kernel (elementwise.hip): item = (t, slot) < T (H + 2 KV); reads
     qkv[t][slot][0, HD), the RoPE row positions[t]; writes q / k / v (and the low halves)."""
     S = H + 2 * KV
     a.span("qk_norm_rope", qkv, 0, T * S * HD * F32)
@@ -244,7 +244,7 @@ def vt_rows(a, kernel, vt, rows, vt_cols, vcol_used):
 
 
 def qkv_norm_rope_vt(a, T, H, KV, HD, qkv16, positions, q, k, v, vcol, vt_cols, vt, vc):
-    """qkv_norm_rope_vt_kernel (elementwise.hip:417): token t = 64 blockIdx + 4 wave + i < T; V^T rows
+    """qkv_norm_rope_vt_kernel (elementwise.hip): token t = 64 blockIdx + 4 wave + i < T; V^T rows
     r < KV HD at column vcol[t] for t < T."""
     S = H + 2 * KV
     a.span("qkv_norm_rope_vt", qkv16, 0, T * S * HD * F16)
@@ -256,7 +256,7 @@ def qkv_norm_rope_vt(a, T, H, KV, HD, qkv16, positions, q, k, v, vcol, vt_cols, 
 
 
 def v_transpose(a, T, width, v, vcol, vt_cols, vt, vc):
-    """v_transpose_kernel (attention.hip:1294): reads v[t][c0 + cc .. + 8) for t < T, c0 + cc < width;
+    """v_transpose_kernel (attention.hip): reads v[t][c0 + cc .. + 8) for t < T, c0 + cc < width;
     writes vt[c0 + d][vcol[t]]."""
     a.span("v_transpose", v, 0, T * width * F16)
     a.span("v_transpose", vcol, 0, T * I32)
@@ -267,9 +267,9 @@ EPI_BYTES = {"f32": lambda N: N * F32, "f16": lambda N: N * F16, "geglu": lambda
 
 
 def gemm(a, kernel, M, N, K, x, y, epi):
-    """launch_gemm_q8 (gemm.hip:698): gemm_kernel (:259) or gemm_skinny_kernel (:295). The activation
+    """launch_gemm_q8 (gemm.hip): gemm_kernel or gemm_skinny_kernel. The activation
     resource covers X[M][K] (buffer_rsrc(X, M K 2)); stores are guarded by row < M, col < N
-    (gemm_store_tile, :81), the GeGLU pairs writing column gcol / 2 of N / 2."""
+    (gemm_store_tile), the GeGLU pairs writing column gcol / 2 of N / 2."""
     if M == 0:
         return
     a.rsrc(kernel, x, 0, M * K * F16)
@@ -277,8 +277,8 @@ def gemm(a, kernel, M, N, K, x, y, epi):
 
 
 def gemm_qkv(a, M, N, K, hd, H, KV, x, e, pos, vc):
-    """launch_gemm_qkv (gemm.hip:734): short batches take the skinny GEMM into the fp16 staging
-    [M][N] and qkv_rowpass_kernel (:553), else gemm_qkv_kernel (:441); both read positions[t] and
+    """launch_gemm_qkv (gemm.hip): short batches take the skinny GEMM into the fp16 staging
+    [M][N] and qkv_rowpass_kernel, else gemm_qkv_kernel; both read positions[t] and
     vcol[t] for t < M, store q / k / v rows t < M and V^T rows (slot - H - KV) HD + d at vcol[t]."""
     if M == 0:
         return
@@ -296,8 +296,8 @@ def gemm_qkv(a, M, N, K, hd, H, KV, x, e, pos, vc):
 
 def attention_items(a, kernel, work, H, KV, HD, q, k, vt, vt_cols, o, item_queries, q_lo=None, k_lo=None,
                     leave_empty=True):
-    """attention_v2_kernel (attention.hip:291), attention_v3_kernel (:556, one workgroup per KV head or per query head) and
-    attention_split_kernel (:860): per work item (seq_start, len, q0, vt_start) with len > 0 and head h, resources
+    """attention_v2_kernel (attention.hip), attention_v3_kernel (one workgroup per KV head or per query head) and
+    attention_split_kernel: per work item (seq_start, len, q0, vt_start) with len > 0 and head h, resources
         Q at (seq_start qStride + h HD) of ((len - 1) qStride + HD) halves, K likewise over kvStride,
         V^T at (kvh HD vt_cols + vt_start) of ((HD - 1) vt_cols + vt_cols - vt_start) halves,
     and output stores at row seq_start + qi for qi < min(q0 + item_queries, len). The kernels leave
@@ -324,7 +324,7 @@ def attention_items(a, kernel, work, H, KV, HD, q, k, vt, vt_cols, o, item_queri
 
 
 def attention_legacy(a, work, H, KV, HD, hw, q, k, v, o, rows_alloc_k):
-    """attention_kernel (attention.hip:93) with attn_stage (:52): plain loads of q rows qi < len, K and
+    """attention_kernel (attention.hip) with attn_stage: plain loads of q rows qi < len, K and
     V key rows kb .. kb + 63 of every 64-key block from the window start (not clamped to the
     sequence: the callers keep 64 rows of slack), output rows qi < len."""
     w = work[work[:, 1] > 0]
@@ -345,14 +345,14 @@ def attention_legacy(a, work, H, KV, HD, hw, q, k, v, o, rows_alloc_k):
 
 
 def pooled_projection(a, n_rows, width, n_out, x, out):
-    """pooled_projection_kernel (elementwise.hip:630): rows r < n_rows of x [*][width] (16-byte loads
+    """pooled_projection_kernel (elementwise.hip): rows r < n_rows of x [*][width] (16-byte loads
     of columns clamped to width - 4), out[r][n] for n < n_out. The weight planes are the model's."""
     a.span("pooled_projection", x, 0, n_rows * width * F32)
     a.span("pooled_projection", out, 0, n_rows * n_out * F32)
 
 
 def mean_pool(a, seqs, width, x, seq_ptr, pooled):
-    """mean_pool_kernel (elementwise.hip:562): rows start .. start + len - 1 of each sequence, 16-byte
+    """mean_pool_kernel (elementwise.hip): rows start .. start + len - 1 of each sequence, 16-byte
     loads of columns c .. c + 3 < width."""
     a.span("mean_pool", seq_ptr, 0, len(seqs) * SEQ_BYTES)
     a.span("mean_pool", pooled, 0, len(seqs) * width * F32)
@@ -457,7 +457,7 @@ def replay(m, b, positions=None):
                                                         (rs, F32)])
                 ple_t = rows("ple_t", r0, m["pl"], F32)
                 gemm(a, "gemm_ple_gate", T, m["pl"], D, x16, ple_t, "f32")
-                # ple_gate_kernel (ple.hip:171) reads ple[(row L + layer) pl .. + pl) of its part's rows
+                # ple_gate_kernel (ple.hip) reads ple[(row L + layer) pl .. + pl) of its part's rows
                 row_kernel(a, "ple_gate", T, [(ple_t, m["pl"] * F32), (rs, F32), (rows("g16", r0, m["pl"], F16), m["pl"] * F16),
                                               (rows("rs2", r0, 1, F32), F32)])
                 if T:
