@@ -1480,8 +1480,15 @@ void trace(ge_ctx* c, const char* name, int layer, float* out, size_t cap, size_
 // queue a new stream gets depends on every stream of the process, so each candidate is tried: a
 // kernel that ends on it while a longer one (a bounded spin) runs on `beside` shows another queue.
 // A candidate on the same queue leaves the next one on another, so two nearly always do; on a busy
-// device, where no candidate shows it, the last one is taken.
+// device, where no candidate shows it, the last one is taken. The waits concern these streams alone, so
+// they also run while another part of the program captures a graph (in HIP's global mode, which would refuse
+// them to every thread and end that capture).
 hipStream_t concurrent_stream(hipStream_t beside) {
+    struct RelaxedCapture {
+        hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+        RelaxedCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+        ~RelaxedCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+    } relaxed;
     constexpr int kTries = 4;
     constexpr int kSpinUs = 300;
     hipEvent_t long_end = nullptr;

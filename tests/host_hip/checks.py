@@ -239,3 +239,12 @@ def test_packs_split_only_into_parts_worth_a_stream(tmp_path, lengths, parts):
             model.context.forward([[5] * n for n in lengths])
     rows = [n for _, n in seen]
     assert len(rows) == parts and sum(rows) == sum(lengths) and min(rows) * 8 >= sum(lengths)
+
+
+def test_a_context_is_created_beside_a_capture():
+    """The search for a second hardware queue waits for its own streams: that must not be refused while another
+    part of the program captures a graph, nor end its capture."""
+    lib.host_hip_capture(1)
+    ctx = ge.Context.create(0)
+    assert lib.host_hip_capture(0) == 1
+    ctx.close()

@@ -5,7 +5,9 @@
 // - every operation is pending from its enqueue until a call waits for it (streams, events and
 //   stream waits are followed with one counter per stream), so a test can ask what a call left
 //   in flight;
-// - a named call can be made to fail.
+// - a named call can be made to fail;
+// - a capture in global mode by another part of the program can be under way: calls that wait or allocate are
+//   then refused, and end that capture, unless their thread has relaxed its mode.
 // One thread at a time.
 #include <hip/hip_runtime_api.h>
 
@@ -15,6 +17,7 @@
 #include <cstring>
 #include <map>
 #include <string>
+#include <utility>
 #include <vector>
 
 struct ihipStream_t {
@@ -42,6 +45,14 @@ std::map<const void*, void*>& vars() {  // host shadow -> block
 std::map<std::string, int> g_fail;  // call -> calls until it fails once
 hipError_t g_last = hipSuccess;      // set by failed launches only
 void (*g_on_launch)(const char*, void**) = nullptr;
+
+bool g_capture = false, g_capture_ended = false;
+hipStreamCaptureMode g_mode = hipStreamCaptureModeGlobal;  // the calling thread's
+// Whether a call that a capture forbids is refused now.
+bool forbidden() {
+    if (!g_capture || g_mode == hipStreamCaptureModeRelaxed) return false;
+    return g_capture_ended = true;
+}
 
 // Streams by id: operations issued, those known complete, and what each stream has waited for.
 std::vector<uint64_t> g_issued, g_done;
@@ -137,6 +148,13 @@ int host_hip_block(const void* p, void** base, size_t* bytes) {
 }
 // The n-th call of `name` from now fails once ("kernel:<part of a kernel's name>" for a launch).
 void host_hip_fail(const char* name, int n) { g_fail[name] = n; }
+// Begins (1) or ends (0) a capture elsewhere in the program; returns whether one that ran was undisturbed.
+int host_hip_capture(int on) {
+    const bool whole = !g_capture_ended;
+    g_capture = on;
+    g_capture_ended = false;
+    return whole && g_mode == hipStreamCaptureModeGlobal;
+}
 void host_hip_on_launch(void (*f)(const char*, void**)) { g_on_launch = f; }
 
 // ---- the calls of the library
@@ -161,7 +179,10 @@ hipError_t hipGetLastError(void) {
     return e;
 }
 
-hipError_t hipMalloc(void** p, size_t n) { return failing("hipMalloc") ? hipErrorOutOfMemory : get_block(p, n); }
+hipError_t hipMalloc(void** p, size_t n) {
+    if (forbidden()) return hipErrorStreamCaptureUnsupported;
+    return failing("hipMalloc") ? hipErrorOutOfMemory : get_block(p, n);
+}
 hipError_t hipFree(void* p) { return p ? drop_block(p) : void(), hipSuccess; }
 hipError_t hipHostMalloc(void** p, size_t n, unsigned) {
     return failing("hipHostMalloc") ? hipErrorOutOfMemory : get_block(p, n);
@@ -195,6 +216,7 @@ hipError_t hipStreamCreateWithFlags(hipStream_t* s, unsigned) {
 }
 hipError_t hipStreamDestroy(hipStream_t s) { return delete s, hipSuccess; }
 hipError_t hipStreamSynchronize(hipStream_t s) {
+    if (forbidden()) return hipErrorStreamCaptureUnsupported;
     if (failing("hipStreamSynchronize")) return hipErrorUnknown;
     merge(g_done, front(id_of(s)));
     return hipSuccess;
@@ -209,16 +231,19 @@ hipError_t hipEventRecord(hipEvent_t e, hipStream_t s) {
     return hipSuccess;
 }
 hipError_t hipEventSynchronize(hipEvent_t e) {
+    if (forbidden()) return hipErrorStreamCaptureUnsupported;
     if (failing("hipEventSynchronize")) return hipErrorUnknown;
     return merge(g_done, e->snap), hipSuccess;
 }
 hipError_t hipEventQuery(hipEvent_t e) {
+    if (forbidden()) return hipErrorStreamCaptureUnsupported;
     for (size_t i = 0; i < e->snap.size(); i++)
         if (e->snap[i] > slot(g_done, i)) return hipErrorNotReady;
     return hipSuccess;
 }
 hipError_t hipEventElapsedTime(float* ms, hipEvent_t, hipEvent_t) { return *ms = 1.0f, hipSuccess; }
 
+hipError_t hipThreadExchangeStreamCaptureMode(hipStreamCaptureMode* m) { return std::swap(*m, g_mode), hipSuccess; }
 hipError_t hipStreamBeginCapture(hipStream_t, hipStreamCaptureMode) { return hipSuccess; }
 hipError_t hipStreamEndCapture(hipStream_t, hipGraph_t* g) { return *g = nullptr, hipSuccess; }
 hipError_t hipGraphInstantiate(hipGraphExec_t* x, hipGraph_t, hipGraphNode_t*, char*, size_t) {
